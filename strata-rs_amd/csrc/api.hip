@@ -28,7 +28,7 @@
 // nothing. Each device holds its own copy until the process ends. Host code
 // never passes `scratch` itself (a host-side name, not a device address):
 // it passes the per-device address from hipGetSymbolAddress.
-constexpr size_t kScratchBytes = size_t(4) << 20;
+constexpr size_t kScratchBytes = sh::kFfnFixedScratch;
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
 namespace {

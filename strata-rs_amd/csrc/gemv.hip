@@ -679,7 +679,7 @@ static hipError_t launch_q8_odd(int nb, const uint8_t* w, int rows, int cols, co
 // ---------------------------------------------------------------- launch --
 // CU count of the current device, queried once per device. The cache is
 // atomic: the entry points are called from several threads at once.
-static int cu_count() {
+int cu_count() {
   constexpr int kDevs = 64;
   static std::atomic<int> cache[kDevs];
   int dev = 0;

@@ -34,6 +34,8 @@ hipError_t launch_silu_mul(const float* g, const float* u, float* h, int64_t n, 
 
 // The dense FFN half of a layer for n_tok tokens (rms_norm, gate, up, silu,
 // down, residual); workspace of ffn_workspace_bytes.
+constexpr size_t kFfnFixedScratch = size_t(4) << 20;  // of sh_ffn_dev_noalloc
+constexpr int64_t kFfnMaxTokTokens = 65535;  // tokens of the many-token form (a grid dimension of its conversion)
 size_t ffn_workspace_bytes(int64_t n_tok, int64_t n_embd, int64_t n_ff);
 hipError_t launch_ffn(uint32_t q_gate, uint32_t q_up, uint32_t q_down, const void* gate, const void* up,
                       const void* down, int q6g, int q6u, int q6d, int64_t n_embd, int64_t n_ff, int n_tok,
@@ -187,6 +189,34 @@ hipError_t launch_quantize_q8(const float* x, int64_t n, int8_t* q, float* scale
 // -> int8 codes, one scale per 256 and the integer code sum per 32.
 hipError_t launch_quantize_q8k(const float* x, int64_t n, int8_t* q, float* scales, int32_t* sums,
                                hipStream_t stream);
+
+// Weight rows against many tokens at the matvecs' precision (tok_mm.hip):
+// prep converts the tokens once into the A fragments of `img`
+// (tok_image_bytes; their order depends on the weights' type), mm writes
+// `nsplit` partial sums out[share][token][ld], which the reader adds in order
+// of the share (tok_sum, or the silu prep of a following product). `rows` is
+// per matrix; two matrices (w1 not null) of one type and shape put w1's rows
+// after w0's.
+struct TokPlan {
+  int tok, groups;          // tokens per group (8, 16, 32, 64, 96), groups
+  int nsb, sb_per, nsplit;  // super-blocks of a row, of a share, shares
+  int tiles;                // 128-row tiles
+};
+bool tok_ok(uint32_t quant, int64_t rows, int64_t cols);
+TokPlan tok_plan(int64_t rows, int mats, int64_t cols, int tokens, int cu, int max_split);
+size_t tok_image_bytes(const TokPlan& p);
+hipError_t launch_tok_prep(const TokPlan& p, uint32_t quant, const float* x, int64_t ld, int cols, int tokens,
+                           void* img, hipStream_t s);
+// The values silu(g) * u from partial sums gu[s][t][ld]: g at [0, cols), u at
+// [cols, 2 cols).
+hipError_t launch_tok_prep_silu(const TokPlan& p, uint32_t quant, const float* gu, int64_t ld, int64_t part,
+                                int nsplit, int cols, int tokens, void* img, hipStream_t s);
+hipError_t launch_tok_mm(const TokPlan& p, uint32_t quant, const void* w0, const void* w1, int64_t rows, int64_t cols,
+                         const void* img, float* out, int64_t ld, int64_t part, int tokens, int reading,
+                         hipStream_t s);
+hipError_t launch_tok_sum(const float* part, int64_t stride, int nsplit, const float* res, float* out, int64_t n,
+                          hipStream_t s);
+int cu_count();  // of the current device
 
 // The trait's elementwise methods over `rows` rows of n floats (rope:
 // head_dim floats per row, row r at position pos0 + r / heads_per_pos).

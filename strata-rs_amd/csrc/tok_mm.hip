@@ -1,0 +1,565 @@
+// Weight rows against many token vectors: y[t][r] = sum_c W[r][c] x[t][c]
+// as `tokens` calls of ops::gemv (crates/strata-core/src/ops.rs:14-28), for
+// 2 tokens to thousands, at the matvecs' precision (tok.hpp's operands).
+//
+// The launches: tok_prep_kernel converts the tokens once per call into the
+// MFMA's A fragments (a super-block of a token group is one contiguous run,
+// the order the matmul's LDS ring takes them in), tok_mm_kernel multiplies,
+// and rows whose columns were split over workgroups are added by the launch
+// that reads them (a fixed order, so results do not depend on timing).
+//
+// tok_mm_kernel: workgroup = 4 waves x 32 weight rows against one token
+// group, over its share of the super-blocks. A wave forms the B fragments of
+// its own 32 rows from registers, each packed byte loaded and decoded once
+// per token group, a super-block ahead; the group's A fragments come
+// through a ring of three LDS buffers (global_load_lds, two stages ahead)
+// that the four waves share. A group is
+//   32, 64 or 96 tokens: hi and lo limbs are fragments of their own, both
+//     added into the same f32 sums (a stage is 64 columns);
+//   8 or 16 tokens: the hi limbs are A rows [0, T) and the lo limbs rows
+//     [T, 2 T) of one fragment, so no matrix work is done for padding at 16
+//     (a stage is a whole super-block).
+// Bound: weights are read and decoded once per group, so few tokens are
+// bound by the weight stream and many by MFMA (two f16 products per weight
+// and token). Per launch in a kernel trace: gate and up of 4096 x 12288 Q4_K
+// (two matrices) 25 us at 24 tokens, 58 us at 77, 285 us at 512 (363 TFLOP/s
+// of x, twice that of f16); down of 12288 x 4096 Q6_K 27, 44 and 244 us (its
+// 16-column sub-blocks cost 16 scalings per MFMA pair).
+// v_mfma_f32_32x32x16_f16: A row / B column = lane % 32, k = 8 (lane / 32) +
+// [0, 8); D column (weight row) = lane % 32, D row (token) = 8 (i / 4) + 4
+// (lane / 32) + i % 4.
+#include <algorithm>
+
+#include "common.hpp"
+#include "kernels.hpp"
+#include "tok.hpp"
+
+namespace sh {
+
+constexpr int kTokRows = 128;  // weight rows per workgroup
+constexpr int kTokThreads = 256;
+
+// The image of a token group's super-block: 16 k steps (pieces per step:
+// tiles x limbs), the sub-block sums of x (one fragment a tile), and the
+// 2^-k of its tokens; whole KiB.
+template <int TOK>
+struct TokShape {
+  static constexpr bool kPacked = TOK <= 16;  // hi and lo limbs in one fragment
+  static constexpr int kTiles = kPacked ? 1 : TOK / 32;
+  static constexpr int kLimbs = kPacked ? 1 : 2;
+  static constexpr int kPiece = TOK == 8 ? 512 : 1024;
+  static constexpr int kGroup = 4 * kTiles * kLimbs * kPiece;  // 64 columns
+  static constexpr int kSums = kTiles * kPiece;
+  static constexpr int kSb = 4 * kGroup + kSums + (TOK == 8 ? 512 : 1024);
+};
+constexpr int tok_sb_bytes(int tok) {
+  return tok == 8 ? TokShape<8>::kSb : tok == 16 ? TokShape<16>::kSb : tok == 32 ? TokShape<32>::kSb
+       : tok == 64 ? TokShape<64>::kSb : TokShape<96>::kSb;
+}
+
+// Byte of piece (row m of the fragment, lane half h): a fragment of 32 rows
+// (16 at 8 tokens, whose rows 16 to 31 repeat them and are not used).
+__device__ __forceinline__ int tok_row_byte(int tok, int m, int h) { return ((tok == 8 ? 16 : 32) * h + m) * 16; }
+
+// ------------------------------------------------------------------- prep --
+// A wave per (token, super-block): lane l holds columns 4 l .. 4 l + 3.
+// SILU: the values are silu(g) * u of the partial sums g = sum_s part[s][t]
+// [c], u = sum_s part[s][t][cols + c] (ops.rs:85-87, in order of s), else
+// x[t][c]. Columns past the row are zero.
+struct TokPrep {
+  const float* x;
+  int64_t ld;    // floats between tokens of x (or of a partial sum)
+  int64_t part;  // floats between partial sums
+  int nsplit;
+  int cols, nsb, tokens, tok, perm;
+  uint8_t* img;
+};
+
+template <bool SILU>
+__global__ void __launch_bounds__(256) tok_prep_kernel(TokPrep a) {
+  const int lane = threadIdx.x & 63;
+  const int sb = blockIdx.x * 4 + (threadIdx.x >> 6), t = blockIdx.y;
+  if (sb >= a.nsb) return;
+  const int c0 = 256 * sb + 4 * lane;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  if (c0 < a.cols) {  // whole 4-column pieces: cols is a multiple of 32
+    const float* p = a.x + int64_t(t) * a.ld + c0;
+    v = *reinterpret_cast<const f32x4*>(p);
+    if constexpr (SILU) {
+      f32x4 u = *reinterpret_cast<const f32x4*>(p + a.cols);
+      for (int s = 1; s < a.nsplit; ++s) {
+        v += *reinterpret_cast<const f32x4*>(p + s * a.part);
+        u += *reinterpret_cast<const f32x4*>(p + s * a.part + a.cols);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = v[k] / (1.f + expf(-v[k])) * u[k];
+    }
+  }
+  float m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+  float s = (v.x + v.y) + (v.z + v.w);
+#pragma unroll
+  for (int off = 1; off < 8; off <<= 1) {
+    m = fmaxf(m, __shfl_xor(m, off, kWave));
+    s += __shfl_xor(s, off, kWave);
+  }
+#pragma unroll
+  for (int off = 8; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, kWave));
+  // 2^k with max |x| 2^k in [2^14, 2^15); a maximum that is not finite makes
+  // every sum of the token NaN (a NaN element does so by itself)
+  int e = 0;
+  (void)frexpf(m, &e);
+  const int k = m > 0.f ? min(15 - e, 126) : 0;
+  const float up = ldexpf(1.f, k);
+  const float down = (m - m == 0.f) ? ldexpf(1.f, -k) : __builtin_nanf("");
+
+  const int tok = a.tok;
+  const int group = t / tok, tg = t - group * tok;  // this token in its group
+  const bool packed = tok <= 16;
+  const int tile = packed ? 0 : tg >> 5, row = packed ? tg : tg & 31;
+  const int tiles = packed ? 1 : tok / 32, limbs = packed ? 1 : 2;
+  const int piece = tok == 8 ? 512 : 1024;
+  const int gbytes = 4 * tiles * limbs * piece;
+  uint8_t* base = a.img + (int64_t(group) * a.nsb + sb) * tok_sb_bytes(tok);
+
+  f16x2_t h01, h23, l01, l23;  // columns (0, 2) and (1, 3): tok.hpp's slot order
+  const float y0 = v.x * up, y1 = v.y * up, y2 = v.z * up, y3 = v.w * up;
+  h01[0] = static_cast<_Float16>(y0);
+  h01[1] = static_cast<_Float16>(y2);
+  h23[0] = static_cast<_Float16>(y1);
+  h23[1] = static_cast<_Float16>(y3);
+  l01[0] = static_cast<_Float16>(y0 - static_cast<float>(h01[0]));
+  l01[1] = static_cast<_Float16>(y2 - static_cast<float>(h01[1]));
+  l23[0] = static_cast<_Float16>(y1 - static_cast<float>(h23[0]));
+  l23[1] = static_cast<_Float16>(y3 - static_cast<float>(h23[1]));
+
+  const int j = lane >> 3, c = (4 * lane) & 31;  // sub-block, column in it
+  const int i = a.perm ? c >> 4 : (c >> 3) & 1, half = a.perm ? (c >> 3) & 1 : c >> 4;
+  const int step = 2 * (j & 1) + i;
+  uint8_t* p = base + (j >> 1) * gbytes + (tile * 4 + step) * limbs * piece + 2 * (c & 7);
+  const u32x2 hi = {__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23)};
+  const u32x2 lo = {__builtin_bit_cast(uint32_t, l01), __builtin_bit_cast(uint32_t, l23)};
+  *reinterpret_cast<u32x2*>(p + tok_row_byte(tok, row, half)) = hi;
+  if (packed)
+    *reinterpret_cast<u32x2*>(p + tok_row_byte(tok, row + tok, half)) = lo;
+  else
+    *reinterpret_cast<u32x2*>(p + piece + tok_row_byte(tok, row, half)) = lo;
+
+  // sub-block sums of x as hi and lo of sum * 2^(k - 5), against the mins in
+  // both lane halves: apart in the k slots, or (packed) in the A rows
+  uint8_t* sums = base + 4 * gbytes + tile * piece;
+  if ((lane & 7) == 0) {
+    const float y = ldexpf(s, k - 5);
+    const _Float16 sh = static_cast<_Float16>(y), sl = static_cast<_Float16>(y - static_cast<float>(sh));
+    *reinterpret_cast<_Float16*>(sums + tok_row_byte(tok, row, 0) + 2 * j) = sh;
+    if (packed) {
+      *reinterpret_cast<_Float16*>(sums + tok_row_byte(tok, row + tok, 0) + 2 * j) = sl;
+      *reinterpret_cast<_Float16*>(sums + tok_row_byte(tok, row, 1) + 2 * j) = _Float16(0);
+      *reinterpret_cast<_Float16*>(sums + tok_row_byte(tok, row + tok, 1) + 2 * j) = _Float16(0);
+    } else {
+      *reinterpret_cast<_Float16*>(sums + tok_row_byte(tok, row, 1) + 2 * j) = sl;
+    }
+  }
+  if (lane == 0) reinterpret_cast<float*>(base + 4 * gbytes + tiles * piece)[tg] = down;
+}
+
+// ----------------------------------------------------------------- matmul --
+struct TokMm {
+  const uint8_t *w0, *w1;  // two matrices of the same shape (w1 null: one)
+  int rows, tiles;         // rows of each, 128-row tiles of both
+  int64_t rb;              // bytes per row
+  int nsb, sb_per, nsplit; // super-blocks of a row, of a workgroup's share, shares
+  int nblk;                // 32-column blocks of a row
+  const uint8_t* img;
+  float* out;              // [nsplit][tokens][ld]; w1's rows follow w0's
+  int64_t ld, part;        // floats between tokens, between shares
+  int tokens, groups, q6s;
+};
+
+template <class F, int TOK>
+__global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
+  using S = TokShape<TOK>;
+  constexpr int NT = S::kTiles;
+  constexpr int kAcc = TOK == 8 ? 8 : 16;  // D values of a tile that are used
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int r32 = lane & 31, half = lane >> 5;
+
+  // workgroup -> (share, 8 row tiles, token group, row tile): the groups of
+  // a row tile run on one XCD (workgroup i on XCD i % 8), near in time, and
+  // share the weights in its L2
+  int id = blockIdx.x;
+  const int t8 = id & 7;
+  id >>= 3;
+  const int group = id % a.groups;
+  id /= a.groups;
+  const int nt8 = (a.tiles + 7) >> 3;
+  const int share = id / nt8, tile = (id - share * nt8) * 8 + t8;
+  if (tile >= a.tiles) return;
+  const int per_mat = a.w1 ? a.tiles >> 1 : a.tiles;
+  const int mat = tile >= per_mat;
+  const int row0 = (tile - mat * per_mat) * kTokRows + 32 * wave;
+  const int sb0 = share * a.sb_per, n = min(a.sb_per, a.nsb - sb0);
+  const uint8_t* wr = (mat ? a.w1 : a.w0) + int64_t(min(row0 + r32, a.rows - 1)) * a.rb + int64_t(sb0) * F::kSbBytes;
+  const uint8_t* img = a.img + (int64_t(group) * a.nsb + sb0) * S::kSb;
+  const int blk0 = a.nblk - 8 * sb0;  // blocks from this share's first
+
+  typename F::Raw raw0, raw1;  // even and odd super-blocks: no copies between them
+  typename F::Sb sb;
+  f32x16_t y[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) y[t] = f32x16_t{};
+
+  // one 64-column group: its k steps into acc (kSub 0, over the super-block)
+  // or scaled by sub-block into acc
+  auto group_mma = [&](auto G, const uint8_t* A, f32x16_t (&acc)[NT], int left) {
+    constexpr int g = decltype(G)::value;
+    TokFrag f[4];
+    F::template frags<g>(sb, f);
+    float sc[4];
+    F::template sub<g>(sb, sc, a.q6s, left);
+    auto frag_a = [&](int t, int k, int limb) {
+      const int at = TOK == 8 ? (16 * half + (lane & 15)) * 16 : 16 * lane;
+      return *reinterpret_cast<const f16x8_t*>(A + ((t * 4 + k) * S::kLimbs + limb) * S::kPiece + at);
+    };
+    if constexpr (F::kSub == 0) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int limb = 0; limb < S::kLimbs; ++limb)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag_a(t, k, limb), f[k].v, acc[t], 0, 0, 0);
+    } else {
+      // unit u = (k steps of a sub-block, tile): its MFMAs go out before unit
+      // u - 1's sums are scaled, so the two overlap and only two units' sums
+      // are held (the barriers keep the compiler from batching the MFMAs)
+      constexpr int kSteps = F::kSub == 1 ? 1 : 2, kUnits = 4 / kSteps * NT;
+      f32x16_t dd[2];
+#pragma unroll
+      for (int u = 0; u <= kUnits; ++u) {
+        if (u < kUnits) {
+          const int k = u / NT * kSteps, t = u % NT;
+          f32x16_t v = {};
+#pragma unroll
+          for (int k2 = 0; k2 < kSteps; ++k2)
+#pragma unroll
+            for (int limb = 0; limb < S::kLimbs; ++limb)
+              v = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag_a(t, k + k2, limb), f[k + k2].v, v, 0, 0, 0);
+          dd[u & 1] = v;
+        }
+        if (u > 0) {
+          const int t = (u - 1) % NT;
+#pragma unroll
+          for (int i = 0; i < kAcc; ++i) acc[t][i] = __builtin_fmaf(dd[(u - 1) & 1][i], sc[(u - 1) / NT], acc[t][i]);
+          asm volatile("" : "+v"(acc[t]));  // here and not where the sums are used
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  // a super-block's sums into y: y += 2^-k (d acc - dmin 2^5 mn)
+  auto finish_sb = [&](const uint8_t* sums, f32x16_t (&acc)[NT]) {
+    const float d = F::d(sb);
+    const float* pk = reinterpret_cast<const float*>(sums + S::kSums);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      f32x16_t mn = {};
+      float dm = 0.f;
+      if constexpr (F::kMin) {
+        dm = -32.f * F::dmin(sb);
+        const int at = TOK == 8 ? (16 * half + (lane & 15)) * 16 : 16 * lane;
+        mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const f16x8_t*>(sums + t * S::kPiece + at),
+                                                    F::mins(sb), mn, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i4 = 0; i4 < kAcc / 4; ++i4) {
+        const int tk = TOK == 8 ? 4 * half : TOK == 16 ? 8 * (i4 & 1) + 4 * half : 32 * t + 8 * i4 + 4 * half;
+        const f32x4 p = *reinterpret_cast<const f32x4*>(pk + tk);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float v = d * acc[t][4 * i4 + i];
+          if constexpr (F::kMin) v = __builtin_fmaf(dm, mn[4 * i4 + i], v);
+          y[t][4 * i4 + i] = __builtin_fmaf(p[i], v, y[t][4 * i4 + i]);
+        }
+      }
+    }
+  };
+  auto load_sb = [&](int s, auto G, typename F::Raw& raw) {
+    const int sc = min(s, n - 1);
+    F::template load<decltype(G)::value>(wr + int64_t(sc) * F::kSbBytes, half, raw, blk0 - 8 * sc);
+    asm volatile("" ::: "memory");  // the loads stay here, a super-block ahead of their use
+  };
+  using std::integral_constant;
+  const integral_constant<int, 0> g0;
+  const integral_constant<int, 1> g1;
+  const integral_constant<int, 2> g2;
+  const integral_constant<int, 3> g3;
+
+  if constexpr (S::kPacked) {
+    // stage = super-block: kCopies copies a wave (past the image: its last
+    // KiB again, the same bytes to the same place)
+    constexpr int kKib = S::kSb / 1024, kCopies = (kKib + 3) / 4;
+    auto stage = [&](int s, int slot) {
+      const uint8_t* src = img + int64_t(min(s, n - 1)) * S::kSb;
+      uint8_t* dst = lds + slot * S::kSb;
+#pragma unroll
+      for (int k = 0; k < kCopies; ++k) {
+        const int q = min(wave + 4 * k, kKib - 1);
+        copy16_to_lds(src + q * 1024 + 16 * lane, dst + q * 1024);
+      }
+    };
+    load_sb(0, g0, raw0);
+    load_sb(0, g1, raw0);
+    load_sb(0, g2, raw0);
+    load_sb(0, g3, raw0);
+    stage(0, 0);
+    stage(1, 1);
+    wait_vmem<kCopies>();
+    int slot = 0;
+    auto super_block = [&](int s, typename F::Raw& cur, typename F::Raw& next) {
+      // weights of s and stage s have landed when no more than the newest
+      // kCopies operations, stage s + 1's copies, are outstanding. The next
+      // weights go out ahead of the next copies: a wait for them with copies
+      // behind would be a wait for everything (the compiler counts no vector
+      // memory operation past a pending LDS copy)
+      wait_vmem<kCopies>();
+      lds_barrier();
+      load_sb(s + 1, g0, next);
+      load_sb(s + 1, g1, next);
+      load_sb(s + 1, g2, next);
+      load_sb(s + 1, g3, next);
+      stage(s + 2, slot == 0 ? 2 : slot - 1);
+      const uint8_t* A = lds + slot * S::kSb;
+      const int left = blk0 - 8 * s;
+      f32x16_t acc[NT] = {};
+      F::template take<0>(cur, sb);
+      group_mma(g0, A, acc, left);
+      F::template take<1>(cur, sb);
+      group_mma(g1, A + S::kGroup, acc, left);
+      F::template take<2>(cur, sb);
+      group_mma(g2, A + 2 * S::kGroup, acc, left);
+      F::template take<3>(cur, sb);
+      group_mma(g3, A + 3 * S::kGroup, acc, left);
+      finish_sb(A + 4 * S::kGroup, acc);
+      slot = slot == 2 ? 0 : slot + 1;
+    };
+    for (int s = 0; s < n; s += 2) {
+      super_block(s, raw0, raw1);
+      if (s + 1 < n) super_block(s + 1, raw1, raw0);
+    }
+  } else {
+    // stage = 64 columns: 2 NT copies a wave; the sums and 2^-k of a
+    // super-block go to an area of their own in its first stage
+    constexpr int kCopies = 2 * NT;
+    uint8_t* tail = lds + 3 * S::kGroup;
+    auto stage = [&](int c, int slot) {
+      const int cc = min(c, 4 * n - 1);
+      const uint8_t* src = img + int64_t(cc >> 2) * S::kSb + (cc & 3) * S::kGroup;
+      uint8_t* dst = lds + slot * S::kGroup;
+#pragma unroll
+      for (int k = 0; k < kCopies; ++k) {
+        const int q = wave + 4 * k;
+        copy16_to_lds(src + q * 1024 + 16 * lane, dst + q * 1024);
+      }
+    };
+    load_sb(0, g0, raw0);
+    load_sb(0, g1, raw0);
+    load_sb(0, g2, raw0);
+    load_sb(0, g3, raw0);
+    stage(0, 0);
+    stage(1, 1);
+    wait_vmem<kCopies>();
+    int slot = 0;
+    auto super_block = [&](int s, typename F::Raw& cur, typename F::Raw& next) {
+      f32x16_t acc[NT] = {};
+      const int left = blk0 - 8 * s;
+      auto step = [&](auto G) {
+        constexpr int g = decltype(G)::value;
+        // stage 4 s + g has landed when no more than the newest kCopies
+        // operations are outstanding; every wave is past the slot that the
+        // next copies overwrite
+        wait_vmem<kCopies>();
+        lds_barrier();
+        if constexpr (g == 0) {
+          const int q = min(wave, NT);  // NT fragments and one KiB of 2^-k
+          copy16_to_lds(img + int64_t(s) * S::kSb + 4 * S::kGroup + q * 1024 + 16 * lane, tail + q * 1024);
+        }
+        stage(4 * s + g + 2, slot == 0 ? 2 : slot - 1);
+        F::template take<g>(cur, sb);
+        load_sb(s + 1, G, next);
+        group_mma(G, lds + slot * S::kGroup, acc, left);
+        slot = slot == 2 ? 0 : slot + 1;
+      };
+      step(g0);
+      step(g1);
+      step(g2);
+      step(g3);
+      finish_sb(tail, acc);
+    };
+    for (int s = 0; s < n; s += 2) {
+      super_block(s, raw0, raw1);
+      if (s + 1 < n) super_block(s + 1, raw1, raw0);
+    }
+  }
+
+  wait_vmem<0>();  // no copy into this workgroup's LDS outlives it
+  // ---- the share's sums
+  const int r = row0 + r32;
+  if (r >= a.rows) return;
+  float* o = a.out + share * a.part + int64_t(mat) * a.rows + r;
+  const int tg0 = group * TOK;
+  if constexpr (S::kPacked) {
+#pragma unroll
+    for (int i = 0; i < TOK / 2; ++i) {
+      const int t = tg0 + (TOK == 8 ? 4 * half + i : 8 * (i >> 2) + 4 * half + (i & 3));
+      if (t < a.tokens) o[int64_t(t) * a.ld] = y[0][i] + y[0][i + TOK / 2];
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int tk = tg0 + 32 * t + 8 * (i >> 2) + 4 * half + (i & 3);
+        if (tk < a.tokens) o[int64_t(tk) * a.ld] = y[t][i];
+      }
+  }
+}
+
+// out[i] = res[i] + sum_s part[s][i], in order of s (res optional); V floats
+// a thread.
+template <int V>
+__global__ void __launch_bounds__(256) tok_sum_kernel(const float* __restrict__ part, int64_t stride, int nsplit,
+                                                      const float* res, float* out, int64_t n) {
+  typedef float vec __attribute__((ext_vector_type(V)));
+  const int64_t i = V * (blockIdx.x * int64_t(blockDim.x) + threadIdx.x);
+  if (i >= n) return;
+  vec v = *reinterpret_cast<const vec*>(part + i);
+  for (int s = 1; s < nsplit; ++s) v += *reinterpret_cast<const vec*>(part + s * stride + i);
+  if (res) v = *reinterpret_cast<const vec*>(res + i) + v;
+  *reinterpret_cast<vec*>(out + i) = v;
+}
+
+// ------------------------------------------------------------------- host --
+bool tok_ok(uint32_t quant, int64_t rows, int64_t cols) {
+  return device_quant(quant) && rows > 0 && rows <= (int64_t(1) << 24) && cols > 0 && cols <= (int64_t(1) << 20) &&
+         cols % geometry(quant).block == 0;
+}
+
+TokPlan tok_plan(int64_t rows, int mats, int64_t cols, int tokens, int cu, int max_split) {
+  TokPlan p{};
+  if (tokens <= 8) {
+    p.tok = 8;
+  } else if (tokens <= 16) {
+    p.tok = 16;
+  } else {
+    const int g = (tokens + 95) / 96;
+    p.tok = ((tokens + g - 1) / g + 31) / 32 * 32;
+  }
+  p.groups = (tokens + p.tok - 1) / p.tok;
+  p.nsb = int((cols + 255) / 256);
+  p.tiles = int((rows + kTokRows - 1) / kTokRows) * mats;
+  // workgroups the chip holds at once: two per CU (LDS) from 64 tokens,
+  // about four below
+  const int64_t slots = int64_t(cu) * (p.tok >= 64 ? 2 : 4);
+  // shares of the columns: the fewest rounds of workgroups, each round as
+  // long as a share plus about two super-blocks of start and end
+  double best = 0;
+  for (int s = 1; s <= std::min(max_split, p.nsb); ++s) {
+    const int per = (p.nsb + s - 1) / s;
+    if ((p.nsb + per - 1) / per != s) continue;
+    const int64_t wg = int64_t(p.tiles) * p.groups * s;
+    const double t = std::max(1.0, double(wg) / double(slots)) * (per + 2) + 0.25 * s;
+    if (p.nsplit == 0 || t < best) {
+      best = t;
+      p.nsplit = s;
+      p.sb_per = per;
+    }
+  }
+  return p;
+}
+
+size_t tok_image_bytes(const TokPlan& p) { return size_t(p.groups) * p.nsb * size_t(tok_sb_bytes(p.tok)); }
+
+static int tok_perm(uint32_t quant) { return quant == kQ6_K || quant == kIQ4_XS; }
+
+hipError_t launch_tok_prep(const TokPlan& p, uint32_t quant, const float* x, int64_t ld, int cols, int tokens,
+                           void* img, hipStream_t s) {
+  const TokPrep a{x, ld, 0, 1, cols, p.nsb, tokens, p.tok, tok_perm(quant), static_cast<uint8_t*>(img)};
+  hipLaunchKernelGGL(tok_prep_kernel<false>, dim3(unsigned((p.nsb + 3) / 4), unsigned(tokens)), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_tok_prep_silu(const TokPlan& p, uint32_t quant, const float* gu, int64_t ld, int64_t part,
+                                int nsplit, int cols, int tokens, void* img, hipStream_t s) {
+  const TokPrep a{gu, ld, part, nsplit, cols, p.nsb, tokens, p.tok, tok_perm(quant), static_cast<uint8_t*>(img)};
+  hipLaunchKernelGGL(tok_prep_kernel<true>, dim3(unsigned((p.nsb + 3) / 4), unsigned(tokens)), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+template <class F, int TOK>
+static void launch_tok(const TokMm& a, int64_t blocks, hipStream_t s) {
+  using S = TokShape<TOK>;
+  const size_t lds = S::kPacked ? 3 * size_t(S::kSb) : 3 * size_t(S::kGroup) + S::kSums + 1024;
+  hipLaunchKernelGGL((tok_mm_kernel<F, TOK>), dim3(unsigned(blocks)), dim3(kTokThreads), lds, s, a);
+}
+template <class F>
+static void launch_tok_f(int tok, const TokMm& a, int64_t blocks, hipStream_t s) {
+  switch (tok) {
+    case 8: launch_tok<F, 8>(a, blocks, s); break;
+    case 16: launch_tok<F, 16>(a, blocks, s); break;
+    case 32: launch_tok<F, 32>(a, blocks, s); break;
+    case 64: launch_tok<F, 64>(a, blocks, s); break;
+    default: launch_tok<F, 96>(a, blocks, s);
+  }
+}
+
+hipError_t launch_tok_mm(const TokPlan& p, uint32_t quant, const void* w0, const void* w1, int64_t rows, int64_t cols,
+                         const void* img, float* out, int64_t ld, int64_t part, int tokens, int reading,
+                         hipStream_t s) {
+  TokMm a{};
+  a.w0 = static_cast<const uint8_t*>(w0);
+  a.w1 = static_cast<const uint8_t*>(w1);
+  a.rows = int(rows);
+  a.tiles = p.tiles;
+  a.rb = byte_size(quant, cols);
+  a.nsb = p.nsb;
+  a.sb_per = p.sb_per;
+  a.nsplit = p.nsplit;
+  a.nblk = int(cols / 32);
+  a.img = static_cast<const uint8_t*>(img);
+  a.out = out;
+  a.ld = ld;
+  a.part = part;
+  a.tokens = tokens;
+  a.groups = p.groups;
+  a.q6s = reading;
+  const int64_t blocks = int64_t(p.nsplit) * ((p.tiles + 7) / 8) * p.groups * 8;
+  if (blocks > (int64_t(1) << 31) - 1) return hipErrorInvalidValue;
+  switch (quant) {
+    case kQ4_K: launch_tok_f<TokQ4Q5<kQ4_K>>(p.tok, a, blocks, s); break;
+    case kQ5_K: launch_tok_f<TokQ4Q5<kQ5_K>>(p.tok, a, blocks, s); break;
+    case kQ6_K: launch_tok_f<TokQ6>(p.tok, a, blocks, s); break;
+    case kQ8_0: launch_tok_f<TokQ8>(p.tok, a, blocks, s); break;
+    case kIQ4_XS:
+      if (reading) launch_tok_f<TokIQ4<true>>(p.tok, a, blocks, s);
+      else launch_tok_f<TokIQ4<false>>(p.tok, a, blocks, s);
+      break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_tok_sum(const float* part, int64_t stride, int nsplit, const float* res, float* out, int64_t n,
+                          hipStream_t s) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(part) | reinterpret_cast<uintptr_t>(res) |
+                       reinterpret_cast<uintptr_t>(out) | uintptr_t(4 * n) | uintptr_t(4 * stride);
+  if (at & 15u)
+    hipLaunchKernelGGL(tok_sum_kernel<1>, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, part, stride, nsplit, res,
+                       out, n);
+  else
+    hipLaunchKernelGGL(tok_sum_kernel<4>, dim3(unsigned((n / 4 + 255) / 256)), dim3(256), 0, s, part, stride, nsplit,
+                       res, out, n);
+  return hipGetLastError();
+}
+
+}  // namespace sh

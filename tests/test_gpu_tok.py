@@ -1,0 +1,87 @@
+"""Many tokens through the dense FFN (sh_ffn_dev above 8 tokens: tok_mm.hip)
+vs the oracle's sho_dense_ffn, at the sizes where the kernels' tiles end:
+token groups of 16, 32, 64 and 96 and one more than each, row counts that are
+no multiple of the 128-row tiles, columns of one and of several shares, Q8_0
+rows that end inside a 256-column step (odd block counts included), weights
+at 2-byte alignment, every format in each of its readings.
+
+Tolerance: the matvec bars (conftest.check_parity) on out - x. The
+activations are held to 22 bits and every sum is f32, so the result is within
+a few f32 roundings of the oracle's, as the 8-token matvecs are.
+"""
+import numpy as np
+import pytest
+
+import strata_hip as H
+from conftest import check_parity
+from strata_hip import synth as S
+
+pytestmark = pytest.mark.gpu
+Q8_0, Q4_K, Q5_K, Q6_K, IQ4_XS = 8, 12, 13, 14, 23
+
+
+def ffn(quants, flags, mats, n_embd, n_ff, x, norm, offset=0):
+    """offset: bytes between the weights' start and a 256-byte boundary."""
+    import torch
+    dev = []
+    for m in mats:
+        t = torch.zeros(m.nbytes + offset, dtype=torch.uint8, device="cuda")
+        t[offset:] = torch.from_numpy(np.ascontiguousarray(m)).cuda()
+        dev.append(t)
+    xd, nd = torch.from_numpy(np.ascontiguousarray(x)).cuda(), torch.from_numpy(norm).cuda()
+    out = torch.full_like(xd, float("nan"))
+    nb = H.ffn_workspace_bytes(x.shape[0], n_embd, n_ff)
+    ws = torch.full((nb,), 0xFF, dtype=torch.uint8, device="cuda")  # NaNs wherever it is read unwritten
+    H.ffn_dev([(q, f, t.data_ptr() + offset) for q, f, t in zip(quants, flags, dev)], n_embd, n_ff, x.shape[0],
+              xd.data_ptr(), nd.data_ptr(), 1e-6, out.data_ptr(), ws.data_ptr(), nb,
+              torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("quants,n_embd,n_ff,n_tok,offset", [
+    ((Q4_K, Q4_K, Q6_K), 512, 768, 9, 0),
+    ((Q4_K, Q4_K, Q6_K), 768, 1280, 16, 2),
+    ((Q5_K, Q5_K, Q4_K), 768, 1280, 17, 2),
+    ((Q6_K, Q6_K, Q5_K), 1024, 512, 33, 2),
+    ((Q4_K, Q4_K, Q4_K), 256, 256, 64, 0),
+    ((Q8_0, Q8_0, Q6_K), 768, 1280, 65, 0),
+    ((Q6_K, Q6_K, Q6_K), 512, 2816, 96, 0),
+    ((Q4_K, Q4_K, Q8_0), 1024, 768, 97, 0),
+    ((Q5_K, Q5_K, Q5_K), 512, 512, 200, 0),
+    ((Q8_0, Q8_0, Q8_0), 1056, 2080, 13, 0),   # 33 and 65 blocks a row
+    ((Q8_0, Q8_0, Q8_0), 288, 96, 70, 4),
+    ((IQ4_XS, IQ4_XS, Q8_0), 512, 768, 21, 0),
+])
+def test_ffn_many_tokens(oracle, quants, n_embd, n_ff, n_tok, offset):
+    print("[case] ffn tokens", quants, n_embd, n_ff, n_tok, offset, flush=True)
+    mats = [S.matrix(quants[0], 91, n_ff, n_embd), S.matrix(quants[1], 92, n_ff, n_embd),
+            S.matrix(quants[2], 93, n_embd, n_ff)]
+    x = S.normal_f32(94 + n_tok, n_tok * n_embd).reshape(n_tok, n_embd)
+    x[n_tok // 2] *= 100.0     # scales of its own
+    x[1, :32] *= 1e-7          # a block far below the rest of its super-block
+    x[2] = 0.0
+    norm = S.normal_f32(95, n_embd)
+    got = ffn(quants, (0, 0, 0), mats, n_embd, n_ff, x, norm, offset)
+    want = oracle.dense_ffn(quants, mats, n_embd, n_ff, x, norm, 1e-6)
+    for t in range(n_tok):  # a token at a time: each has its own magnitude
+        check_parity(got[t].astype(np.float64) - x[t], want[t].astype(np.float64) - x[t], f"token {t}",
+                     strict_tol=None)
+    rest = [t for t in range(n_tok) if t != n_tok // 2]
+    check_parity(got[rest].astype(np.float64) - x[rest], want[rest].astype(np.float64) - x[rest], "ffn out - x")
+
+
+@pytest.mark.parametrize("quant,flag", [(Q6_K, H.FLAG_Q6K_SIGNED_SCALES), (IQ4_XS, H.FLAG_IQ4XS_GGML)])
+def test_ffn_many_tokens_other_reading(oracle, quant, flag):
+    """The flagged readings, against the oracle on the dequantized rows."""
+    print("[case] ffn tokens, reading", quant, flag, flush=True)
+    n_embd, n_ff, n_tok = 512, 768, 40
+    mats = [S.matrix(quant, 96, n_ff, n_embd), S.matrix(quant, 97, n_ff, n_embd), S.matrix(quant, 98, n_embd, n_ff)]
+    x = S.normal_f32(99, n_tok * n_embd).reshape(n_tok, n_embd)
+    norm = S.normal_f32(100, n_embd)
+    mode = oracle.SCALE_I8 if quant == Q6_K else oracle.IQ4XS_GGML
+    f32 = [oracle.dequantize_row(quant, m, r * c, mode) for m, (r, c) in
+           zip(mats, ((n_ff, n_embd), (n_ff, n_embd), (n_embd, n_ff)))]
+    got = ffn((quant,) * 3, (flag,) * 3, mats, n_embd, n_ff, x, norm)
+    want = oracle.dense_ffn((0, 0, 0), [w.view(np.uint8) for w in f32], n_embd, n_ff, x, norm, 1e-6)
+    check_parity(got.astype(np.float64) - x, want.astype(np.float64) - x, "ffn out - x")
