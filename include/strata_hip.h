@@ -277,13 +277,17 @@ int sh_matmul(sh_context* ctx, const sh_quant_tensor* w, const float* x, uint32_
 
 /* ---- device-pointer variants (asynchronous on `stream`) ---------------- */
 
-/* Bytes of device workspace sh_matmul_dev needs. */
+/* Bytes of device workspace sh_matmul_dev uses: the converted activations,
+ * and, where the output's tiles are too few for the chip, the partial sums
+ * of columns split over more workgroups. */
 int sh_matmul_workspace_bytes(uint32_t quant, uint64_t rows, uint64_t cols, uint32_t m, uint32_t mode,
                               uint64_t* bytes);
 
 /* sh_matmul on device pointers: w (4-byte aligned), x [m][cols], y
- * [m][rows], workspace at least sh_matmul_workspace_bytes() long and
- * 256-byte aligned. Calls sharing one workspace must not overlap in time. */
+ * [m][rows], workspace sh_matmul_workspace_bytes() long and
+ * 256-byte aligned (one that holds the activations but not the partial sums
+ * is taken too: such a call splits its columns less or not at all). Calls
+ * sharing one workspace must not overlap in time. */
 int sh_matmul_dev(uint32_t quant, uint32_t flags, const void* w, uint64_t rows, uint64_t cols,
                   const float* x, uint32_t m, float* y, uint32_t mode, void* workspace,
                   uint64_t workspace_bytes, void* stream);

@@ -807,7 +807,7 @@ int sh_matmul(sh_context* c, const sh_quant_tensor* w, const float* x, uint32_t 
   const uint64_t need = rows * uint64_t(sh::byte_size(w->quant, int64_t(cols)));
   if ((rc = resident(c, w->key, w->quant, 1, rows, cols, w->data, need, &r))) return rc;
   const size_t xb = sizeof(float) * cols * m, yb = sizeof(float) * rows * m;
-  const size_t ws = sh::matmul_workspace_bytes(int64_t(cols), int64_t(m), mode);
+  const size_t ws = sh::matmul_workspace_bytes(w->quant, int64_t(rows), int64_t(cols), int64_t(m), mode);
   if ((rc = c->d_in.ensure(xb, "x buffer")) || (rc = c->d_blk.ensure(ws, "workspace")) ||
       (rc = c->h_in.ensure(xb, "x staging")) || (rc = c->h_out.ensure(yb, "y staging")))
     return rc;
@@ -816,7 +816,7 @@ int sh_matmul(sh_context* c, const sh_quant_tensor* w, const float* x, uint32_t 
   // the tiles store y once each: straight into the mapped staging
   HIP_TRY(sh::launch_matmul(w->quant, r->dev, int64_t(rows), int64_t(cols),
                             static_cast<const float*>(c->d_in.p), int64_t(m), static_cast<float*>(c->h_out.dev),
-                            mode, c->d_blk.p, reading(w->quant, w->flags), c->stream),
+                            mode, c->d_blk.p, ws, reading(w->quant, w->flags), c->stream),
           "matmul launch");
   HIP_TRY(hipStreamSynchronize(c->stream), "matmul");
   memcpy(y, c->h_out.p, yb);
@@ -1037,7 +1037,7 @@ int sh_matmul_workspace_bytes(uint32_t quant, uint64_t rows, uint64_t cols, uint
   if (!bytes) return fail(SH_ERR_INVALID_ARGUMENT, "null bytes");
   int rc = matmul_check(quant, rows, cols, m, mode);
   if (rc) return rc;
-  *bytes = sh::matmul_workspace_bytes(int64_t(cols), int64_t(m), mode);
+  *bytes = sh::matmul_workspace_bytes(quant, int64_t(rows), int64_t(cols), int64_t(m), mode);
   return SH_OK;
 }
 
@@ -1047,7 +1047,7 @@ int sh_matmul_dev(uint32_t quant, uint32_t flags, const void* w, uint64_t rows, 
   if (!w || !x || !y || !workspace) return fail(SH_ERR_INVALID_ARGUMENT, "null pointer");
   int rc = matmul_check(quant, rows, cols, m, mode);
   if (rc) return rc;
-  const uint64_t need = sh::matmul_workspace_bytes(int64_t(cols), int64_t(m), mode);
+  const uint64_t need = sh::matmul_workspace_min(int64_t(cols), int64_t(m), mode);
   if (workspace_bytes < need)
     return fail(SH_ERR_INVALID_ARGUMENT, "workspace of %llu bytes, %llu needed",
                 (unsigned long long)workspace_bytes, (unsigned long long)need);
@@ -1055,7 +1055,7 @@ int sh_matmul_dev(uint32_t quant, uint32_t flags, const void* w, uint64_t rows, 
       (reinterpret_cast<uintptr_t>(workspace) & 255u))
     return fail(SH_ERR_INVALID_ARGUMENT, "misaligned pointer (w needs 4 bytes, x 16, workspace 256)");
   HIP_TRY(sh::launch_matmul(quant, w, int64_t(rows), int64_t(cols), x, int64_t(m), y, mode, workspace,
-                            reading(quant, flags), static_cast<hipStream_t>(stream)),
+                            size_t(workspace_bytes), reading(quant, flags), static_cast<hipStream_t>(stream)),
           "matmul launch");
   return SH_OK;
 }

@@ -16,7 +16,8 @@
 //         32-element block, which the VALU scales by the weight block's scale
 //         and the activation block's scale (and subtracts the Q4_K min term).
 //
-// Workgroup tile: 256 tokens x 96 weight rows, K in 64-element chunks.
+// Workgroup tile: 256 (or 128) tokens x 96 weight rows, K in 64-element
+// chunks, the columns split over workgroups where the tiles are few (mm_shape).
 // bf16 (mm_bf16_ws_kernel): 8 waves by role -- 4 consumers (wave w owns
 // tokens [64w, 64w + 64) and all 96 rows: 2 x 3 MFMA tiles of 32 x 32),
 // 3 stagers dequantizing each weight chunk into a double-buffered bf16 LDS
@@ -638,12 +639,14 @@ __global__ void __launch_bounds__(256) x_q8k_tiled_kernel(const float* __restric
 }
 
 // --------------------------------------------------------------- tile order --
+// (blockIdx.y is the share of the columns, if they are split)
+template <int BM = kMmBM>
 __device__ __forceinline__ void tile_of(int n_tiles_m, int& r0, int& t0) {
   int bid = blockIdx.x;
   const int nb = gridDim.x;
   if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
   r0 = (bid / n_tiles_m) * kMmBN;
-  t0 = (bid % n_tiles_m) * kMmBM;
+  t0 = (bid % n_tiles_m) * BM;
 }
 
 // Q6_K piece -> bf16 runs (scale bytes of the runs: hb and 2 + hb)
@@ -728,17 +731,21 @@ constexpr int kMmWsThreads = 512;
 constexpr size_t kMmLdsWs = 2 * kMmBN * kMmRowB;
 constexpr int kBfDepth = 3;  // weight chunks a stager's loads run ahead (4: about 2% slower), Q8_0 / Q6_K
 
-template <class S>
-__global__ void __launch_bounds__(kMmWsThreads)
+template <class S, int MI>
+__global__ void __launch_bounds__(kMmWsThreads, MI == 1 ? 4 : 2)
     mm_bf16_ws_kernel(const uint8_t* __restrict__ w, int n_rows, int cols, int64_t row_bytes,
-                      const u32x4* __restrict__ xt, int m, float* __restrict__ y, int n_tiles_m, int q6s) {
+                      const u32x4* __restrict__ xt, int m, float* __restrict__ y, int n_tiles_m, int q6s,
+                      int c_per, int64_t part) {
   extern __shared__ __attribute__((aligned(16))) uint8_t wlb[];  // [2][kMmBN * kMmRowB]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
   int r0, t0;
-  tile_of(n_tiles_m, r0, t0);
+  tile_of<128 * MI>(n_tiles_m, r0, t0);
   const int nchunks = cols / kMmKC;
+  // this share's chunks [cb, ce): whole super-blocks (c_per is a multiple of 4)
+  const int cb = blockIdx.y * c_per, ce = min(cb + c_per, nchunks);
+  y += blockIdx.y * part;
   const bool consumer = wave < 4, stager = wave >= 4 && wave < 7;
 
   // B staging: lane p = tid - 256 < 192 stages row p / 2, piece p % 2
@@ -772,36 +779,36 @@ __global__ void __launch_bounds__(kMmWsThreads)
   // half h of k-step s holds chunk elements [32 h + 8 s, +8) of token 32 T +
   // l32, T the 32-token tile of M-subtile mi (clamped to the last tile)
   const int n_tt = (m + 31) >> 5;
-  const uint8_t* xtile[2];
+  const uint8_t* xtile[MI];
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi) {
-    const int T = min((t0 + 64 * (wave & 3) + 32 * mi) >> 5, n_tt - 1);
+  for (int mi = 0; mi < MI; ++mi) {
+    const int T = min((t0 + 32 * MI * (wave & 3) + 32 * mi) >> 5, n_tt - 1);
     xtile[mi] = reinterpret_cast<const uint8_t*>(xt) + int64_t(T) * nchunks * 4096 + 16 * lane;
   }
-  bf16x8 afr[2][2][4];  // [chunk parity][mi][s]
+  bf16x8 afr[2][MI][4];  // [chunk parity][mi][s]
   auto load_a = [&](int c, bf16x8 (*dst)[4]) {
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
+    for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
       for (int s = 0; s < 4; ++s)
         dst[mi][s] = *reinterpret_cast<const bf16x8*>(xtile[mi] + int64_t(c) * 4096 + 1024 * s);
   };
-  f32x16 acc[2][3];
+  f32x16 acc[MI][3];
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
+  for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
     for (int ni = 0; ni < 3; ++ni) acc[mi][ni] = f32x16{};
 
   typename S::Raw raw[kRingB];
   if (consumer) {
-    load_a(0, afr[0]);
-    load_a(min(1, nchunks - 1), afr[1]);
+    load_a(cb, afr[0]);
+    load_a(min(cb + 1, ce - 1), afr[1]);
   } else if (stager) {
 #pragma unroll
-    for (int k = 0; k < kRingB; ++k) raw[k] = S::load(wrow, min(k, nchunks - 1), piece);
+    for (int k = 0; k < kRingB; ++k) raw[k] = S::load(wrow, min(cb + k, ce - 1), piece);
     if constexpr (kSb) S::sb_scales(raw[0].h, sd, sm);
-    stage(raw[0], 0, wlb, 0);
-    raw[0] = S::load(wrow, min(kRingB, nchunks - 1), piece);
+    stage(raw[0], cb, wlb, 0);
+    raw[0] = S::load(wrow, min(cb + kRingB, ce - 1), piece);
   }
   lds_barrier();
 
@@ -816,7 +823,7 @@ __global__ void __launch_bounds__(kMmWsThreads)
   if (consumer) {
     auto consume = [&](int c, bf16x8 (*a)[4]) {
       const uint8_t* wb = wlb + (c & 1) * (kMmBN * kMmRowB);
-      const int cnext = min(c + 2, nchunks - 1);
+      const int cnext = min(c + 2, ce - 1);
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         bf16x8 bfr[3];
@@ -824,7 +831,7 @@ __global__ void __launch_bounds__(kMmWsThreads)
         for (int ni = 0; ni < 3; ++ni)
           bfr[ni] = *reinterpret_cast<const bf16x8*>(wb + (32 * ni + l32) * kMmRowB + 2 * (32 * half + 8 * s));
 #pragma unroll
-        for (int mi = 0; mi < 2; ++mi)
+        for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
           for (int ni = 0; ni < 3; ++ni)
             acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[mi][s], bfr[ni], acc[mi][ni], 0, 0, 0);
@@ -833,25 +840,25 @@ __global__ void __launch_bounds__(kMmWsThreads)
         // consumers' loads would otherwise reach the CU's memory pipe in one
         // burst at the chunk's end and stall at issue
 #pragma unroll
-        for (int mi = 0; mi < 2; ++mi)
+        for (int mi = 0; mi < MI; ++mi)
           a[mi][s] = *reinterpret_cast<const bf16x8*>(xtile[mi] + int64_t(cnext) * 4096 + 1024 * s);
-        __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);  // the step's 6 MFMAs,
-        __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);  // then its 2 loads
+        __builtin_amdgcn_sched_group_barrier(0x008, 3 * MI, 0);  // the step's MFMAs,
+        __builtin_amdgcn_sched_group_barrier(0x020, MI, 0);      // then its loads
       }
       lds_barrier();
     };
-    int c0 = 0;
-    for (; c0 + 2 <= nchunks; c0 += 2) {
+    int c0 = cb;
+    for (; c0 + 2 <= ce; c0 += 2) {
       consume(c0, afr[0]);
       consume(c0 + 1, afr[1]);
     }
-    if (c0 < nchunks) consume(c0, afr[0]);
+    if (c0 < ce) consume(c0, afr[0]);
   } else if (stager) {
-    for (int c0 = 0; c0 < nchunks; c0 += kRingB) {
+    for (int c0 = cb; c0 < ce; c0 += kRingB) {
 #pragma unroll
       for (int j = 0; j < kRingB; ++j) {
         const int c = c0 + j;
-        if (c < nchunks) {  // uniform
+        if (c < ce) {  // uniform
           // B(c + 1) into the buffer chunk c - 1 used; past the last chunk
           // this re-stages the last one into the buffer nobody reads (for
           // the K-quants with the next super-block's scales: harmless)
@@ -860,28 +867,28 @@ __global__ void __launch_bounds__(kMmWsThreads)
           // is pair (j + 1) & 3 of its super-block, and j = 3 starts the next
           if constexpr (kSb)
             if (j == kRingB - 1) S::sb_scales(raw[slot].h, sd, sm);
-          stage(raw[slot], min(c + 1, nchunks - 1), wlb + ((c + 1) & 1) * (kMmBN * kMmRowB), (j + 1) & 3);
-          raw[slot] = S::load(wrow, min(c + 1 + kRingB, nchunks - 1), piece);
+          stage(raw[slot], min(c + 1, ce - 1), wlb + ((c + 1) & 1) * (kMmBN * kMmRowB), (j + 1) & 3);
+          raw[slot] = S::load(wrow, min(c + 1 + kRingB, ce - 1), piece);
           lds_barrier();
         }
       }
     }
   } else {
-    for (int c = 0; c < nchunks; ++c) lds_barrier();
+    for (int c = cb; c < ce; ++c) lds_barrier();
   }
 
   if (!consumer) return;
   // D layout of the 32x32 MFMA: lane l holds column l % 32 (a weight row)
   // and, in register i, row 8 * (i / 4) + 4 * (l / 32) + i % 4 (a token)
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi)
+  for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
     for (int ni = 0; ni < 3; ++ni) {
       const int r = r0 + 32 * ni + l32;
       if (r >= n_rows) continue;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int t = t0 + 64 * wave + 32 * mi + 8 * (i >> 2) + 4 * half + (i & 3);
+        const int t = t0 + 32 * MI * wave + 32 * mi + 8 * (i >> 2) + 4 * half + (i & 3);
         if (t < m) y[int64_t(t) * n_rows + r] = acc[mi][ni][i];
       }
     }
@@ -916,16 +923,15 @@ __global__ void __launch_bounds__(kMmWsThreads)
 // others still finish chunk c. Waves 0-2 also stage: at the start of chunk c
 // the codes of chunk c + 1 with d_rj per block, and per super-block
 // (double-buffered) the rows' m_j as bf16 and dmin.
-constexpr int kMiThreads = 512;
 constexpr int kI8Depth = 4;  // chunks per unrolled loop body
 constexpr int kI8Ring = 2;   // weight chunks in flight ahead of staging (register slots)
 constexpr int kI8Bufs = 3;   // chunk tiles in LDS
 
-template <class S>
-__global__ void __launch_bounds__(kMiThreads)
+template <class S, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, 2)
     mm_i8_kernel(const uint8_t* __restrict__ w, int n_rows, int cols, int64_t row_bytes,
                  const int8_t* __restrict__ xq, const float* __restrict__ xs, const u32x4* __restrict__ xu,
-                 int m, float* __restrict__ y, int n_tiles_m) {
+                 int m, float* __restrict__ y, int n_tiles_m, int c_per, int64_t part) {
   typedef float f32x32 __attribute__((ext_vector_type(32)));
   constexpr bool kMin = S::kMin;
   __shared__ __attribute__((aligned(16))) uint8_t wl[kI8Bufs][kMmBN * kMmRowQ];  // [chunk buf] codes
@@ -936,12 +942,15 @@ __global__ void __launch_bounds__(kMiThreads)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
   int r0, t0;
-  tile_of(n_tiles_m, r0, t0);
+  tile_of<32 * WAVES>(n_tiles_m, r0, t0);
   const int nchunks = cols / kMmKC;
+  // this share's chunks [cb, ce): whole super-blocks (c_per is a multiple of 4)
+  const int cb = blockIdx.y * c_per, ce = min(cb + c_per, nchunks);
+  y += blockIdx.y * part;
   const int nblk = cols / 32, nsb = cols >> 8;
 
   constexpr int kTasks = kMmBN * S::kPieces;
-  static_assert(kTasks % kWave == 0 && kTasks <= kMiThreads, "staging tasks fill whole waves");
+  static_assert(kTasks % kWave == 0 && kTasks <= 64 * WAVES, "staging tasks fill whole waves");
   const bool stager = tid < kTasks;
   const int srow = stager ? tid / S::kPieces : 0, piece = tid % S::kPieces;
   const uint8_t* wrow = w + int64_t(min(r0 + srow, n_rows - 1)) * row_bytes;
@@ -993,17 +1002,18 @@ __global__ void __launch_bounds__(kMiThreads)
   static_assert(kI8Depth % kI8Ring == 0, "ring slots are constants of the unrolled loop");
   typename S::Raw raw[kI8Ring];
 #pragma unroll
-  for (int k = 0; k < kI8Ring; ++k) raw[k] = S::load(wrow, min(k, nchunks - 1), piece);
-  if (stager) stage(raw[0], 0, 0);
-  raw[0] = S::load(wrow, min(kI8Ring, nchunks - 1), piece);
+  for (int k = 0; k < kI8Ring; ++k) raw[k] = S::load(wrow, min(cb + k, ce - 1), piece);
+  const int buf0 = cb % kI8Bufs;
+  if (stager) stage(raw[0], cb, buf0);
+  raw[0] = S::load(wrow, min(cb + kI8Ring, ce - 1), piece);
   // chunk c's activation fragments and the lane's token scale of block
   // `half` (the B operand of the scale products), loaded a chunk ahead; the
   // min operand a super-block ahead
   i32x4 xc[2];
 #pragma unroll
-  for (int s = 0; s < 2; ++s) xc[s] = *reinterpret_cast<const i32x4*>(xr + 1024 * s);
-  float sxc = sr[32 * half];
-  u32x4 uc = kMin ? ur[0] : u32x4{0u, 0u, 0u, 0u};
+  for (int s = 0; s < 2; ++s) xc[s] = *reinterpret_cast<const i32x4*>(xr + int64_t(cb) * 2048 + 1024 * s);
+  float sxc = sr[32 * (2 * cb + half)];
+  u32x4 uc = kMin ? ur[64 * (cb >> 2)] : u32x4{0u, 0u, 0u, 0u};
   lds_barrier();
 
   // step k of a chunk is (row tile k / 2, block k % 2); its weight
@@ -1024,18 +1034,18 @@ __global__ void __launch_bounds__(kMiThreads)
   static_assert(kI8Depth % 4 == 0, "the super-block position repeats every kI8Depth chunks");
   i32x16 Ib[2];
   f32x32 Sb[2];
-  i32x4 a_nn = ld_a(0, 1);
+  i32x4 a_nn = ld_a(buf0, 1);
   float d_nn = 0.f;
-  Ib[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ld_a(0, 0), xc[0], i32x16{}, 0, 0, 0);
-  Sb[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(ld_d(0, 0), sxc, f32x32{}, 0, 0, 0);
+  Ib[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ld_a(buf0, 0), xc[0], i32x16{}, 0, 0, 0);
+  Sb[0] = __builtin_amdgcn_mfma_f32_32x32x1f32(ld_d(buf0, 0), sxc, f32x32{}, 0, 0, 0);
   __builtin_amdgcn_sched_barrier(0);
 
-  for (int c0 = 0; c0 < nchunks; c0 += kI8Depth) {
+  for (int c0 = cb; c0 < ce; c0 += kI8Depth) {
 #pragma unroll
     for (int jj = 0; jj < kI8Depth; ++jj) {
       const int c = c0 + jj;
-      if (c < nchunks) {  // uniform
-        const bool more = c + 1 < nchunks;
+      if (c < ce) {  // uniform
+        const bool more = c + 1 < ce;
         const int buf = c % kI8Bufs, nbuf = (c + 1) % kI8Bufs;
         {
           const int slot = (jj + 1) % kI8Ring;  // chunk c + 1 (a constant once unrolled)
@@ -1044,7 +1054,7 @@ __global__ void __launch_bounds__(kMiThreads)
           // row r0, one cache line a wave): with loads on the stagers' path
           // only, the compiler's counted wait for the activation loads would
           // also wait for these, a whole memory latency each chunk
-          raw[slot] = S::load(wrow, min(c + 1 + kI8Ring, nchunks - 1), piece);
+          raw[slot] = S::load(wrow, min(c + 1 + kI8Ring, ce - 1), piece);
         }
         const int cn = more ? c + 1 : c;
         i32x4 xn[2];
@@ -1155,7 +1165,6 @@ __global__ void __launch_bounds__(kMiThreads)
 // tokens [32 w, +32) x all 96 rows); waves 0-2 stage chunk c + 1 (codes
 // q - 32 as int8, d * sc per sub-block) while chunk c is computed, with a
 // two-chunk ring of weight loads.
-constexpr int kM6Threads = 512;
 
 // Four 6-bit codes q (one per byte) -> the bytes q - 32 (int8, -32..31)
 // without carries between bytes: q ^ 32 clears bit 5 of q >= 32 (giving
@@ -1166,10 +1175,11 @@ __device__ __forceinline__ uint32_t q6_centered(uint32_t q) {
   return t | (m << 1) | (m << 2);
 }
 
-__global__ void __launch_bounds__(kM6Threads)
+template <int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, 2)
     mm_i8q6_kernel(const uint8_t* __restrict__ w, int n_rows, int cols, int64_t row_bytes,
                    const int8_t* __restrict__ xq, const float* __restrict__ xs, int m, float* __restrict__ y,
-                   int n_tiles_m, int q6s) {
+                   int n_tiles_m, int q6s, int c_per, int64_t part) {
   typedef float f32x32 __attribute__((ext_vector_type(32)));
   __shared__ __attribute__((aligned(16))) uint8_t wl[2][kMmBN * kMmRowQ];  // [chunk buf] codes q - 32
   __shared__ __attribute__((aligned(16))) float wsc[2][4][kMmBN];          // [chunk buf][sub-block][row] d * sc
@@ -1177,12 +1187,15 @@ __global__ void __launch_bounds__(kM6Threads)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
   int r0, t0;
-  tile_of(n_tiles_m, r0, t0);
+  tile_of<32 * WAVES>(n_tiles_m, r0, t0);
   const int nchunks = cols / kMmKC;
+  // this share's chunks [cb, ce): whole super-blocks (c_per is a multiple of 4)
+  const int cb = blockIdx.y * c_per, ce = min(cb + c_per, nchunks);
+  y += blockIdx.y * part;
   const int nblk = cols / 32;
 
   constexpr int kTasks = kMmBN * StQ6K::kPieces;
-  static_assert(kTasks % kWave == 0 && kTasks <= kM6Threads, "staging tasks fill whole waves");
+  static_assert(kTasks % kWave == 0 && kTasks <= 64 * WAVES, "staging tasks fill whole waves");
   const bool stager = tid < kTasks;
   const int srow = stager ? tid / StQ6K::kPieces : 0, piece = tid % StQ6K::kPieces;
   const uint8_t* wrow = w + int64_t(min(r0 + srow, n_rows - 1)) * row_bytes;
@@ -1218,29 +1231,29 @@ __global__ void __launch_bounds__(kM6Threads)
   // loop body); every wave issues them (other lanes read row r0), as in
   // mm_i8_kernel
   StQ6K::Raw raw[2];
-  raw[0] = StQ6K::load(wrow, 0, piece);
-  raw[1] = StQ6K::load(wrow, min(1, nchunks - 1), piece);
-  if (stager) stage(raw[0], 0, 0);
-  raw[0] = StQ6K::load(wrow, min(2, nchunks - 1), piece);
+  raw[0] = StQ6K::load(wrow, cb, piece);
+  raw[1] = StQ6K::load(wrow, min(cb + 1, ce - 1), piece);
+  if (stager) stage(raw[0], cb, 0);
+  raw[0] = StQ6K::load(wrow, min(cb + 2, ce - 1), piece);
   i32x4 xc[2];
   float sxc[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    xc[s] = *reinterpret_cast<const i32x4*>(xr + 1024 * s);
-    sxc[s] = sr[32 * s];
+    xc[s] = *reinterpret_cast<const i32x4*>(xr + int64_t(cb) * 2048 + 1024 * s);
+    sxc[s] = sr[32 * (2 * cb + s)];
   }
   lds_barrier();
 
-  for (int c0 = 0; c0 < nchunks; c0 += 2) {
+  for (int c0 = cb; c0 < ce; c0 += 2) {
 #pragma unroll
     for (int jj = 0; jj < 2; ++jj) {
       const int c = c0 + jj;
-      if (c < nchunks) {  // uniform
+      if (c < ce) {  // uniform
         const int buf = c & 1;
-        const bool more = c + 1 < nchunks;
+        const bool more = c + 1 < ce;
         // stage chunk c + 1 (slot (jj + 1) % 2) and refill the slot with c + 3
         if (more && stager) stage(raw[(jj + 1) & 1], c + 1, buf ^ 1);
-        raw[(jj + 1) & 1] = StQ6K::load(wrow, min(c + 3, nchunks - 1), piece);
+        raw[(jj + 1) & 1] = StQ6K::load(wrow, min(c + 3, ce - 1), piece);
         // chunk c + 1's activations, a chunk ahead
         const int cn = more ? c + 1 : c;
         i32x4 xn[2];
@@ -1561,6 +1574,11 @@ __global__ void __launch_bounds__(kMqThreads)
 // -------------------------------------------------------------------- host --
 static size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
+constexpr int kMmMaxShares = 16;
+static size_t mm_part_bytes(int64_t rows, int64_t m, int shares) {
+  return size_t(shares) * sizeof(float) * size_t(rows) * size_t(m);
+}
+
 // Modes: 0 bf16; 1 q8 (activations in 32-element Q8 blocks, every int8
 // format); 2 q8k (activations in 256-element blocks, one scale per weight
 // super-block: Q4_K / Q5_K only; a coarser rounding than mode 1, kept as an
@@ -1614,25 +1632,86 @@ static Q8kWs q8k_ws(uint8_t* ws, int64_t cols, int64_t m) {
   return r;
 }
 
-size_t matmul_workspace_bytes(int64_t cols, int64_t m, uint32_t mode) {
+static size_t mm_act_bytes(int64_t cols, int64_t m, uint32_t mode) {
   if (mode == 0) return align256(size_t((m + 31) / 32 * 32) * size_t(cols) * 2);  // whole 32-token tiles
   if (mode == 2) return q8k_ws(nullptr, cols, m).bytes;
   return q8_ws(nullptr, cols, m).bytes;
 }
 
+// The launch shape: tokens per workgroup (256, or 128 with two workgroups on
+// a CU) and shares of the columns, whose sums the workspace holds after the
+// activations and tok_sum adds in order of the share (few tokens or few rows
+// make fewer tiles than the chip has CUs). Chosen by the time that rounds of
+// workgroups take: a share's chunks plus about six of start and end, each
+// `chunk` us (measured: a 256-token workgroup or two 128-token ones on a CU,
+// or one 128-token one alone), then the sum of the shares at about 4 TB/s.
+// Measured, before (256 tokens, one share) and now: q8 Q5_K 4096 x 12288,
+// 333 tokens 251 -> 104 us; q8 Q6_K 2048 x 4096, 200 tokens 183 -> 42; bf16
+// Q4_K 4096 x 12288, 100 tokens 110 -> 32; bf16 Q6_K 2048 x 2048, 40 tokens
+// 35 -> 16; bf16 Q4_K 12288 x 4096, 512 tokens (256 tiles): one share, as it
+// was. The rule's choice was within 5% of the best of a sweep of both tile
+// heights and 1 to 16 shares over ten shapes.
+struct MmShape {
+  int bm, shares, c_per;  // c_per: chunks of a share, whole super-blocks
+};
+static MmShape mm_shape(uint32_t quant, int64_t rows, int64_t cols, int64_t m, uint32_t mode, size_t room) {
+  const int nch = int(cols / kMmKC);
+  MmShape best{kMmBM, 1, (nch + 3) / 4 * 4};
+  if (mode == 2) return best;
+  const int64_t cu = cu_count(), rt = (rows + kMmBN - 1) / kMmBN;
+  const double part_us = double(m) * double(rows) * 8.0 / 4e6;  // a share's sums written and read
+  double best_t = 0;
+  for (int bm = kMmBM; bm >= kMmBM / 2; bm /= 2) {
+    const int64_t tiles = rt * ((m + bm - 1) / bm);
+    for (int s = 1; s <= kMmMaxShares; ++s) {
+      const int per = ((nch + s - 1) / s + 3) / 4 * 4;
+      if ((nch + per - 1) / per != s) continue;
+      if (s > 1 && mm_part_bytes(rows, m, s) > room) break;
+      const int64_t wg = tiles * s, slots = bm == kMmBM ? cu : 2 * cu;
+      const bool full = bm == kMmBM || wg > cu;
+      const double chunk = mode == 0 ? (full ? 0.8 : 0.5) : quant == kQ6_K ? (full ? 2.8 : 2.1) : (full ? 1.3 : 0.9);
+      const double t = double((wg + slots - 1) / slots) * (per + 6) * chunk + (s > 1 ? 3.0 + s * part_us : 0.0);
+      if (best_t == 0 || t < best_t) {
+        best_t = t;
+        best = {bm, s, per};
+      }
+    }
+  }
+  return best;
+}
+
+size_t matmul_workspace_min(int64_t cols, int64_t m, uint32_t mode) { return mm_act_bytes(cols, m, mode); }
+
+size_t matmul_workspace_bytes(uint32_t quant, int64_t rows, int64_t cols, int64_t m, uint32_t mode) {
+  const size_t act = mm_act_bytes(cols, m, mode);
+  const MmShape sh = mm_shape(quant, rows, cols, m, mode, ~size_t(0));
+  return act + (sh.shares > 1 ? mm_part_bytes(rows, m, sh.shares) : 0);
+}
+
 template <class S>
-static void launch_mm(uint32_t mode, const uint8_t* w, int rows, int cols, int64_t rb, uint8_t* ws, int m,
-                      float* y, int q6s, hipStream_t s) {
-  const int ntm = (m + kMmBM - 1) / kMmBM, ntn = (rows + kMmBN - 1) / kMmBN;
-  const dim3 grid(unsigned(ntm * ntn));
+static void launch_mm(uint32_t mode, const MmShape& sh, const uint8_t* w, int rows, int cols, int64_t rb, uint8_t* ws,
+                      int m, float* y, int q6s, hipStream_t s) {
+  const int ntm = (m + sh.bm - 1) / sh.bm, ntn = (rows + kMmBN - 1) / kMmBN;
+  const dim3 grid(unsigned(ntm * ntn), unsigned(sh.shares));
+  const int64_t part = sh.shares > 1 ? int64_t(m) * rows : 0;
+  const bool wide = sh.bm == kMmBM;
   if (mode == 0) {
-    hipLaunchKernelGGL(mm_bf16_ws_kernel<S>, grid, dim3(kMmWsThreads), kMmLdsWs, s, w, rows, cols, rb,
-                       reinterpret_cast<const u32x4*>(ws), m, y, ntm, q6s);
+    const auto* xt = reinterpret_cast<const u32x4*>(ws);
+    if (wide)
+      hipLaunchKernelGGL((mm_bf16_ws_kernel<S, 2>), grid, dim3(kMmWsThreads), kMmLdsWs, s, w, rows, cols, rb, xt, m, y,
+                         ntm, q6s, sh.c_per, part);
+    else
+      hipLaunchKernelGGL((mm_bf16_ws_kernel<S, 1>), grid, dim3(kMmWsThreads), kMmLdsWs, s, w, rows, cols, rb, xt, m, y,
+                         ntm, q6s, sh.c_per, part);
   } else if constexpr (std::is_same<S, StQ6K>::value) {
     if (mode == 1) {  // 16-element scales: the Q6_K int8 kernel
       const Q8Ws q = q8_ws(ws, cols, m);
-      hipLaunchKernelGGL(mm_i8q6_kernel, grid, dim3(kM6Threads), 0, s, w, rows, cols, rb, q.codes, q.scales, m, y,
-                         ntm, q6s);
+      if (wide)
+        hipLaunchKernelGGL(mm_i8q6_kernel<8>, grid, dim3(512), 0, s, w, rows, cols, rb, q.codes, q.scales, m, y, ntm,
+                           q6s, sh.c_per, part);
+      else
+        hipLaunchKernelGGL(mm_i8q6_kernel<4>, grid, dim3(256), 0, s, w, rows, cols, rb, q.codes, q.scales, m, y, ntm,
+                           q6s, sh.c_per, part);
     }
   } else if constexpr (S::kQ8) {
     if (mode == 2) {
@@ -1643,8 +1722,13 @@ static void launch_mm(uint32_t mode, const uint8_t* w, int rows, int cols, int64
       }
     } else {
       const Q8Ws q = q8_ws(ws, cols, m);
-      hipLaunchKernelGGL(mm_i8_kernel<S>, grid, dim3(kMiThreads), 0, s, w, rows, cols, rb, q.codes, q.scales,
-                         reinterpret_cast<const u32x4*>(q.u), m, y, ntm);
+      const auto* u = reinterpret_cast<const u32x4*>(q.u);
+      if (wide)
+        hipLaunchKernelGGL((mm_i8_kernel<S, 8>), grid, dim3(512), 0, s, w, rows, cols, rb, q.codes, q.scales, u, m, y,
+                           ntm, sh.c_per, part);
+      else
+        hipLaunchKernelGGL((mm_i8_kernel<S, 4>), grid, dim3(256), 0, s, w, rows, cols, rb, q.codes, q.scales, u, m, y,
+                           ntm, sh.c_per, part);
     }
   }
 }
@@ -1668,9 +1752,12 @@ hipError_t launch_quantize_q8k(const float* x, int64_t n, int8_t* q, float* scal
 }
 
 hipError_t launch_matmul(uint32_t quant, const void* wv, int64_t rows, int64_t cols, const float* x,
-                         int64_t m, float* y, uint32_t mode, void* workspace, int q6_signed,
-                         hipStream_t s) {
+                         int64_t m, float* y, uint32_t mode, void* workspace, size_t workspace_bytes,
+                         int q6_signed, hipStream_t s) {
   if (!matmul_shape_ok(quant, rows, cols, m, mode)) return hipErrorInvalidValue;
+  const size_t act = mm_act_bytes(cols, m, mode);
+  if (workspace_bytes < act) return hipErrorInvalidValue;
+  const MmShape sh = mm_shape(quant, rows, cols, m, mode, workspace_bytes - act);
   const uint8_t* w = static_cast<const uint8_t*>(wv);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   const int64_t rb = byte_size(quant, cols);
@@ -1691,18 +1778,21 @@ hipError_t launch_matmul(uint32_t quant, const void* wv, int64_t rows, int64_t c
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
+  float* out = sh.shares > 1 ? reinterpret_cast<float*>(ws + act) : y;
   switch (quant) {
-    case kQ4_K: launch_mm<StQ4K>(mode, w, int(rows), int(cols), rb, ws, int(m), y, q6_signed, s); break;
-    case kQ5_K: launch_mm<StQ5K>(mode, w, int(rows), int(cols), rb, ws, int(m), y, q6_signed, s); break;
-    case kQ8_0: launch_mm<StQ8>(mode, w, int(rows), int(cols), rb, ws, int(m), y, q6_signed, s); break;
-    case kQ6_K: launch_mm<StQ6K>(mode, w, int(rows), int(cols), rb, ws, int(m), y, q6_signed, s); break;
+    case kQ4_K: launch_mm<StQ4K>(mode, sh, w, int(rows), int(cols), rb, ws, int(m), out, q6_signed, s); break;
+    case kQ5_K: launch_mm<StQ5K>(mode, sh, w, int(rows), int(cols), rb, ws, int(m), out, q6_signed, s); break;
+    case kQ8_0: launch_mm<StQ8>(mode, sh, w, int(rows), int(cols), rb, ws, int(m), out, q6_signed, s); break;
+    case kQ6_K: launch_mm<StQ6K>(mode, sh, w, int(rows), int(cols), rb, ws, int(m), out, q6_signed, s); break;
     case kIQ4_XS:  // the reading (reference or ggml qs bytes) is a template argument
-      if (q6_signed) launch_mm<StIQ4XS<true>>(mode, w, int(rows), int(cols), rb, ws, int(m), y, 0, s);
-      else launch_mm<StIQ4XS<false>>(mode, w, int(rows), int(cols), rb, ws, int(m), y, 0, s);
+      if (q6_signed) launch_mm<StIQ4XS<true>>(mode, sh, w, int(rows), int(cols), rb, ws, int(m), out, 0, s);
+      else launch_mm<StIQ4XS<false>>(mode, sh, w, int(rows), int(cols), rb, ws, int(m), out, 0, s);
       break;
     default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
+  e = hipGetLastError();
+  if (e != hipSuccess || sh.shares == 1) return e;
+  return launch_tok_sum(out, m * rows, sh.shares, nullptr, y, m * rows, s);
 }
 
 }  // namespace sh
