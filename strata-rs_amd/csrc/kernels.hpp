@@ -41,10 +41,12 @@ hipError_t launch_ffn(uint32_t q_gate, uint32_t q_up, uint32_t q_down, const voi
                       const void* down, int q6g, int q6u, int q6d, int64_t n_embd, int64_t n_ff, int n_tok,
                       const float* x, const float* post_norm, double eps, float* out, void* workspace,
                       hipStream_t stream);
-// The same for F32 / F16 / BF16 rows against bf16(x) (rounded as loaded).
+constexpr int kPlainMaxBatch = 1024;
+// The same for F32 / F16 / BF16 rows against bf16(x) (rounded as loaded), for
+// up to kPlainMaxBatch vectors.
 hipError_t launch_gemv_plain_bf16x(uint32_t quant, const void* w, int64_t rows, int64_t cols, const float* x,
                                    float* y, int batch, hipStream_t stream);
-// Both in one launch: y1 = W1 . bf16(x) (rows1 rows) and y2 = W2 . x (rows2
+// Both in one launch (up to kPlainMaxBatch vectors): y1 = W1 . bf16(x) (rows1 rows) and y2 = W2 . x (rows2
 // rows of the same type and width), e.g. a MoE layer's router and gate input.
 hipError_t launch_gemv_plain_pair(uint32_t quant, const void* w1, int64_t rows1, const void* w2, int64_t rows2,
                                   int64_t cols, const float* x, float* y1, float* y2, int batch, hipStream_t stream);
@@ -102,6 +104,11 @@ struct MoePlan {
   bool staged;                   // row bytes allow 16-byte tile copies
   bool out_major;                // expert stacks [n_expert][out][in] (moe_om.hip)
   int om_rows_a, om_rows_b;      // out-major: rows per workgroup of gate/up and of down
+  // out-major stacks and many tokens (moe_tok.hip): pairs per work item (0:
+  // not this form), the pairs' tokens and their places in the items, the
+  // fragments of the pairs' x, then of their silu(h) * p
+  int tok;
+  size_t o_pairtok, o_pairslot, o_img;
   // one token over in-major stacks (moe_one.hip): per phase the 64-column
   // units of a column block, column blocks, row slots, rows per chunk,
   // chunks, and threads per column in the row-slot reduction
@@ -125,6 +132,14 @@ bool moe_plan_out_major(int n_tok, int top_k, int n_expert, int n_embd, int n_ff
 void launch_moe_out_major(const MoePlan& p, uint32_t qg, uint32_t qd, const void* gate, const void* up,
                           const void* down, int q6g, int q6u, int q6d, const float* logits, const float* x,
                           void* workspace, bool fused_route, hipStream_t s);
+// The many-token form over out-major stacks: moe_tok_group sets p.tok where
+// it serves the shape better; the launches after the routing.
+int moe_tok_group(const MoePlan& p, uint32_t q_gateup, uint32_t q_down);
+size_t moe_tok_image_bytes(const MoePlan& p);
+struct MoeShared;
+hipError_t launch_moe_tok(const MoePlan& p, uint32_t qg, uint32_t qd, const void* gate, const void* up,
+                          const void* down, int q6g, int q6u, int q6d, const float* x, float* out, void* workspace,
+                          hipStream_t s, const MoeShared* shared);
 // The shared expert's part of the layer's combine: out[t] += sigmoid(s[t])
 // * d[t] after the routed sum, once `join` (if any) has completed.
 struct MoeShared {
@@ -166,6 +181,9 @@ struct MoeLayerPlan {
   MoePlan moe;
   int n_ff_sh;
   size_t o_logits, o_xb, o_g, o_u, o_h, o_d, o_s;  // [n_tok][...] f32 each
+  // the shared expert on tok_mm.hip (sh_tok): its fragments and shares' sums
+  bool sh_tok;
+  size_t o_sh_img, o_sh_part;
   size_t bytes;
 };
 bool moe_layer_plan(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, int n_ff_sh,
@@ -205,18 +223,26 @@ struct TokPlan {
   int nsb, sb_per, nsplit;  // super-blocks of a row, of a share, shares
   int tiles;                // 128-row tiles
 };
+// Groups that are the tokens of one expert each: group i < *n multiplies its
+// cnt[i] tokens (values off[i] .. of the call) with expert e[i]'s matrix,
+// `stride` bytes after its predecessor's.
+struct TokItems {
+  const int *e, *off, *cnt, *n;
+  int64_t stride;
+};
 bool tok_ok(uint32_t quant, int64_t rows, int64_t cols);
 TokPlan tok_plan(int64_t rows, int mats, int64_t cols, int tokens, int cu, int max_split);
 size_t tok_image_bytes(const TokPlan& p);
 hipError_t launch_tok_prep(const TokPlan& p, uint32_t quant, const float* x, int64_t ld, int cols, int tokens,
-                           void* img, hipStream_t s);
+                           void* img, hipStream_t s, const int* src = nullptr, const int* slot = nullptr);
 // The values silu(g) * u from partial sums gu[s][t][ld]: g at [0, cols), u at
 // [cols, 2 cols).
 hipError_t launch_tok_prep_silu(const TokPlan& p, uint32_t quant, const float* gu, int64_t ld, int64_t part,
-                                int nsplit, int cols, int tokens, void* img, hipStream_t s);
+                                int nsplit, int cols, int tokens, void* img, hipStream_t s,
+                                const int* slot = nullptr);
 hipError_t launch_tok_mm(const TokPlan& p, uint32_t quant, const void* w0, const void* w1, int64_t rows, int64_t cols,
                          const void* img, float* out, int64_t ld, int64_t part, int tokens, int reading,
-                         hipStream_t s);
+                         hipStream_t s, const TokItems* items = nullptr);
 hipError_t launch_tok_sum(const float* part, int64_t stride, int nsplit, const float* res, float* out, int64_t n,
                           hipStream_t s);
 int cu_count();  // of the current device

@@ -18,7 +18,10 @@
 // a gate-input row of the same plain type shares its launch. The matvecs are
 // the library's gemv kernels (F32 / F16 / BF16 rows sum in f64 as ops::gemv
 // does; Q8_0 / Q4_K / Q6_K on the integer-limb path), up to 8 tokens per
-// launch.
+// launch for quantized rows; the shared expert of more than 8 tokens runs on
+// tok_mm.hip.
+#include <algorithm>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -47,6 +50,8 @@ hipError_t launch_silu_mul(const float* g, const float* u, float* h, int64_t n, 
   return hipGetLastError();
 }
 
+constexpr int kShMaxSplit = 8;  // shares of the shared expert's columns
+
 static size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
 bool moe_layer_plan(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, int n_ff_sh,
@@ -74,22 +79,54 @@ bool moe_layer_plan(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, in
   p.o_h = take(sizeof(float) * T * n_ff_sh);
   p.o_d = take(sizeof(float) * T * n_embd);
   p.o_s = take(sizeof(float) * T);
+  // the readings (q6 flags) of gate and up are looked at by the launch
+  p.sh_tok = n_tok > 8 && q.gate_sh == q.up_sh && tok_ok(q.gate_sh, n_ff_sh, n_embd) &&
+             tok_ok(q.down_sh, n_embd, n_ff_sh);
+  if (p.sh_tok) {
+    const TokPlan gu = tok_plan(n_ff_sh, 2, n_embd, n_tok, cu_count(), kShMaxSplit);
+    const TokPlan dn = tok_plan(n_embd, 1, n_ff_sh, n_tok, cu_count(), kShMaxSplit);
+    p.o_sh_img = take(std::max(tok_image_bytes(gu), tok_image_bytes(dn)));
+    // as for kShMaxSplit shares, whatever the plans take: more tokens never
+    // need less
+    p.o_sh_part = take(kShMaxSplit * sizeof(float) * T * std::max(2 * n_ff_sh, n_embd));
+  }
   p.bytes = o;
   p.n_ff_sh = n_ff_sh;
   *plan = p;
   return true;
 }
 
+// The shared expert for more than 8 tokens, its weights read once for up to
+// 96 of them (the matvecs: once per 8): d = down . (silu(g) * u).
+static hipError_t shexp_tokens(const MoeLayerPlan& p, const MoeLayerTypes& q, const MoeLayerTensors& w, const float* x,
+                               float* d, uint8_t* ws, hipStream_t s) {
+  const int T = p.moe.n_tok, E = p.moe.n_embd, N = p.n_ff_sh;
+  const TokPlan gu = tok_plan(N, 2, E, T, cu_count(), kShMaxSplit), dn = tok_plan(E, 1, N, T, cu_count(), kShMaxSplit);
+  uint8_t* img = ws + p.o_sh_img;
+  float* part = reinterpret_cast<float*>(ws + p.o_sh_part);
+  const int64_t ng = int64_t(T) * 2 * N, nd = int64_t(T) * E;
+  hipError_t e;
+  if ((e = launch_tok_prep(gu, q.gate_sh, x, E, E, T, img, s)) != hipSuccess) return e;
+  if ((e = launch_tok_mm(gu, q.gate_sh, w.gate_sh, w.up_sh, N, E, img, part, 2 * N, ng, T, w.q6_gate_sh, s)) !=
+      hipSuccess)
+    return e;
+  if ((e = launch_tok_prep_silu(dn, q.down_sh, part, 2 * N, ng, gu.nsplit, N, T, img, s)) != hipSuccess) return e;
+  float* out = dn.nsplit == 1 ? d : part;
+  if ((e = launch_tok_mm(dn, q.down_sh, w.down_sh, nullptr, E, N, img, out, E, nd, T, w.q6_down_sh, s)) != hipSuccess)
+    return e;
+  return dn.nsplit == 1 ? hipSuccess : launch_tok_sum(part, nd, dn.nsplit, nullptr, d, nd, s);
+}
+
 // y[t] = W . x[t] for t < n_tok, 8 tokens per launch; `xbf16`: W . bf16(x[t])
-// (plain-float W only).
+// (plain-float W only, one launch).
 static hipError_t gemv_tokens(uint32_t quant, const void* w, int rows, int cols, const float* x, float* y,
                               int n_tok, int q6s, hipStream_t s, bool xbf16 = false) {
+  if (xbf16) return launch_gemv_plain_bf16x(quant, w, rows, cols, x, y, n_tok, s);
   for (int t0 = 0; t0 < n_tok; t0 += 8) {
     const int nb = n_tok - t0 < 8 ? n_tok - t0 : 8;
     const float* xt = x + int64_t(t0) * cols;
     float* yt = y + int64_t(t0) * rows;
-    const hipError_t e = xbf16 ? launch_gemv_plain_bf16x(quant, w, rows, cols, xt, yt, nb, s)
-                               : launch_gemv(quant, w, rows, cols, xt, yt, nb, q6s, s);
+    const hipError_t e = launch_gemv(quant, w, rows, cols, xt, yt, nb, q6s, s);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -178,6 +215,8 @@ hipError_t launch_moe_layer(const MoeLayerPlan& p, const MoeLayerTypes& q, const
       if ((r = launch_shexp_one(q.gate_sh, q.down_sh, w.gate_sh, w.up_sh, w.down_sh, n_embd, n_sh, x, g, d,
                                 w.q6_gate_sh, w.q6_down_sh, ss)) != hipSuccess)
         return r;
+    } else if (p.sh_tok && w.q6_gate_sh == w.q6_up_sh) {
+      if ((r = shexp_tokens(p, q, w, x, d, ws, ss)) != hipSuccess) return r;
     } else {
       if ((r = gemv_tokens(q.gate_sh, w.gate_sh, n_sh, n_embd, x, g, T, w.q6_gate_sh, ss)) != hipSuccess) return r;
       if ((r = gemv_tokens(q.up_sh, w.up_sh, n_sh, n_embd, x, u, T, w.q6_up_sh, ss)) != hipSuccess) return r;
@@ -192,12 +231,8 @@ hipError_t launch_moe_layer(const MoeLayerPlan& p, const MoeLayerTypes& q, const
     // waits for the shared expert and adds sigmoid(s) * d after the routed sum
     if (pair_rg) {
       // the router on bf16(x) and the gate-input row on x in one launch
-      for (int t0 = 0; t0 < T; t0 += 8) {
-        const int nb = T - t0 < 8 ? T - t0 : 8;
-        if ((r = launch_gemv_plain_pair(q.router, w.router, E, w.gate_inp, 1, n_embd, x + int64_t(t0) * n_embd,
-                                        logits + int64_t(t0) * E, sg + t0, nb, s)) != hipSuccess)
-          return r;
-      }
+      if ((r = launch_gemv_plain_pair(q.router, w.router, E, w.gate_inp, 1, n_embd, x, logits, sg, T, s)) != hipSuccess)
+        return r;
     } else if (plain_quant(q.router)) {
       if ((r = gemv_tokens(q.router, w.router, E, n_embd, x, logits, T, 0, s, true)) != hipSuccess) return r;
     } else {

@@ -304,7 +304,9 @@ bool moe_plan_out_major(int n_tok, int top_k, int n_expert, int n_embd, int n_ff
   p.rb_b = byte_size(qb, n_ff);
   const int pairs = n_tok * top_k;
   p.s_max = pairs < n_expert ? pairs : n_expert;
-  p.z_max = (pairs + p.s_max + 1) / 2;
+  p.tok = moe_tok_group(p, qa, qb);
+  const int ip = p.tok ? p.tok : 2;  // an expert's pairs, ip to a work item
+  p.z_max = (pairs + p.s_max * (ip - 1)) / ip;
   p.nch_a = p.nch_b = 1;  // whole dot products: one chunk each
   p.om_rows_a = om_rows(n_ff, n_embd, 2, p.s_max);
   p.om_rows_b = om_rows(n_embd, n_ff, 1, p.s_max);
@@ -327,6 +329,11 @@ bool moe_plan_out_major(int n_tok, int top_k, int n_expert, int n_embd, int n_ff
   p.o_item_cnt = take(sizeof(int) * p.z_max);
   p.o_item_tok = take(sizeof(int) * 2 * p.z_max);
   p.o_tokpair = take(sizeof(int) * pairs);
+  if (p.tok) {
+    p.o_pairtok = take(sizeof(int) * pairs);
+    p.o_pairslot = take(sizeof(int) * pairs);
+    p.o_img = take(moe_tok_image_bytes(p));
+  }
   p.o_part_a = take(sizeof(float) * size_t(pairs) * 2 * n_ff);
   p.o_part_b = take(sizeof(float) * size_t(pairs) * n_embd);
   p.bytes = o;

@@ -73,6 +73,8 @@ struct TokPrep {
   int nsplit;
   int cols, nsb, tokens, tok, perm;
   uint8_t* img;
+  const int* src;   // value t is row src[t] of x, and goes to
+  const int* slot;  // place slot[t] of the groups (null: t)
 };
 
 template <bool SILU>
@@ -83,13 +85,14 @@ __global__ void __launch_bounds__(256) tok_prep_kernel(TokPrep a) {
   const int c0 = 256 * sb + 4 * lane;
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
   if (c0 < a.cols) {  // whole 4-column pieces: cols is a multiple of 32
-    const float* p = a.x + int64_t(t) * a.ld + c0;
-    v = *reinterpret_cast<const f32x4*>(p);
+    typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));  // x of any float alignment
+    const float* p = a.x + int64_t(a.src ? a.src[t] : t) * a.ld + c0;
+    v = *reinterpret_cast<const f32x4a4*>(p);
     if constexpr (SILU) {
-      f32x4 u = *reinterpret_cast<const f32x4*>(p + a.cols);
+      f32x4 u = *reinterpret_cast<const f32x4a4*>(p + a.cols);
       for (int s = 1; s < a.nsplit; ++s) {
-        v += *reinterpret_cast<const f32x4*>(p + s * a.part);
-        u += *reinterpret_cast<const f32x4*>(p + s * a.part + a.cols);
+        v += *reinterpret_cast<const f32x4a4*>(p + s * a.part);
+        u += *reinterpret_cast<const f32x4a4*>(p + s * a.part + a.cols);
       }
 #pragma unroll
       for (int k = 0; k < 4; ++k) v[k] = v[k] / (1.f + expf(-v[k])) * u[k];
@@ -113,7 +116,8 @@ __global__ void __launch_bounds__(256) tok_prep_kernel(TokPrep a) {
   const float down = (m - m == 0.f) ? ldexpf(1.f, -k) : __builtin_nanf("");
 
   const int tok = a.tok;
-  const int group = t / tok, tg = t - group * tok;  // this token in its group
+  const int sl = a.slot ? a.slot[t] : t;
+  const int group = sl / tok, tg = sl - group * tok;  // this token in its group
   const bool packed = tok <= 16;
   const int tile = packed ? 0 : tg >> 5, row = packed ? tg : tg & 31;
   const int tiles = packed ? 1 : tok / 32, limbs = packed ? 1 : 2;
@@ -173,6 +177,7 @@ struct TokMm {
   float* out;              // [nsplit][tokens][ld]; w1's rows follow w0's
   int64_t ld, part;        // floats between tokens, between shares
   int tokens, groups, q6s;
+  TokItems items;
 };
 
 template <class F, int TOK>
@@ -190,16 +195,33 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
   int id = blockIdx.x;
   const int t8 = id & 7;
   id >>= 3;
-  const int group = id % a.groups;
-  id /= a.groups;
-  const int nt8 = (a.tiles + 7) >> 3;
-  const int share = id / nt8, tile = (id - share * nt8) * 8 + t8;
-  if (tile >= a.tiles) return;
+  int group, share, tile, p0, cnt;
+  int64_t we = 0;
+  if (a.items.e) {
+    // groups are an expert's tokens: the row tiles of a group run on one
+    // XCD, near in time, and share its fragments in the L2
+    group = id / a.tiles * 8 + t8;
+    tile = id - group / 8 * a.tiles;
+    share = 0;
+    if (group >= *a.items.n) return;
+    we = a.items.e[group] * a.items.stride;
+    p0 = a.items.off[group];
+    cnt = a.items.cnt[group];
+  } else {
+    group = id % a.groups;
+    id /= a.groups;
+    const int nt8 = (a.tiles + 7) >> 3;
+    share = id / nt8;
+    tile = (id - share * nt8) * 8 + t8;
+    if (tile >= a.tiles) return;
+    p0 = group * TOK;
+    cnt = min(TOK, a.tokens - p0);
+  }
   const int per_mat = a.w1 ? a.tiles >> 1 : a.tiles;
   const int mat = tile >= per_mat;
   const int row0 = (tile - mat * per_mat) * kTokRows + 32 * wave;
   const int sb0 = share * a.sb_per, n = min(a.sb_per, a.nsb - sb0);
-  const uint8_t* wr = (mat ? a.w1 : a.w0) + int64_t(min(row0 + r32, a.rows - 1)) * a.rb + int64_t(sb0) * F::kSbBytes;
+  const uint8_t* wr = (mat ? a.w1 : a.w0) + we + int64_t(min(row0 + r32, a.rows - 1)) * a.rb + int64_t(sb0) * F::kSbBytes;
   const uint8_t* img = a.img + (int64_t(group) * a.nsb + sb0) * S::kSb;
   const int blk0 = a.nblk - 8 * sb0;  // blocks from this share's first
 
@@ -406,21 +428,20 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
   // ---- the share's sums
   const int r = row0 + r32;
   if (r >= a.rows) return;
-  float* o = a.out + share * a.part + int64_t(mat) * a.rows + r;
-  const int tg0 = group * TOK;
+  float* o = a.out + share * a.part + int64_t(p0) * a.ld + int64_t(mat) * a.rows + r;
   if constexpr (S::kPacked) {
 #pragma unroll
     for (int i = 0; i < TOK / 2; ++i) {
-      const int t = tg0 + (TOK == 8 ? 4 * half + i : 8 * (i >> 2) + 4 * half + (i & 3));
-      if (t < a.tokens) o[int64_t(t) * a.ld] = y[0][i] + y[0][i + TOK / 2];
+      const int t = TOK == 8 ? 4 * half + i : 8 * (i >> 2) + 4 * half + (i & 3);
+      if (t < cnt) o[int64_t(t) * a.ld] = y[0][i] + y[0][i + TOK / 2];
     }
   } else {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int tk = tg0 + 32 * t + 8 * (i >> 2) + 4 * half + (i & 3);
-        if (tk < a.tokens) o[int64_t(tk) * a.ld] = y[t][i];
+        const int tk = 32 * t + 8 * (i >> 2) + 4 * half + (i & 3);
+        if (tk < cnt) o[int64_t(tk) * a.ld] = y[t][i];
       }
   }
 }
@@ -483,15 +504,16 @@ size_t tok_image_bytes(const TokPlan& p) { return size_t(p.groups) * p.nsb * siz
 static int tok_perm(uint32_t quant) { return quant == kQ6_K || quant == kIQ4_XS; }
 
 hipError_t launch_tok_prep(const TokPlan& p, uint32_t quant, const float* x, int64_t ld, int cols, int tokens,
-                           void* img, hipStream_t s) {
-  const TokPrep a{x, ld, 0, 1, cols, p.nsb, tokens, p.tok, tok_perm(quant), static_cast<uint8_t*>(img)};
+                           void* img, hipStream_t s, const int* src, const int* slot) {
+  const TokPrep a{x, ld, 0, 1, cols, p.nsb, tokens, p.tok, tok_perm(quant), static_cast<uint8_t*>(img), src, slot};
   hipLaunchKernelGGL(tok_prep_kernel<false>, dim3(unsigned((p.nsb + 3) / 4), unsigned(tokens)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_tok_prep_silu(const TokPlan& p, uint32_t quant, const float* gu, int64_t ld, int64_t part,
-                                int nsplit, int cols, int tokens, void* img, hipStream_t s) {
-  const TokPrep a{gu, ld, part, nsplit, cols, p.nsb, tokens, p.tok, tok_perm(quant), static_cast<uint8_t*>(img)};
+                                int nsplit, int cols, int tokens, void* img, hipStream_t s, const int* slot) {
+  const TokPrep a{gu, ld, part, nsplit, cols, p.nsb, tokens, p.tok, tok_perm(quant), static_cast<uint8_t*>(img), nullptr,
+                  slot};
   hipLaunchKernelGGL(tok_prep_kernel<true>, dim3(unsigned((p.nsb + 3) / 4), unsigned(tokens)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
@@ -515,7 +537,7 @@ static void launch_tok_f(int tok, const TokMm& a, int64_t blocks, hipStream_t s)
 
 hipError_t launch_tok_mm(const TokPlan& p, uint32_t quant, const void* w0, const void* w1, int64_t rows, int64_t cols,
                          const void* img, float* out, int64_t ld, int64_t part, int tokens, int reading,
-                         hipStream_t s) {
+                         hipStream_t s, const TokItems* items) {
   TokMm a{};
   a.w0 = static_cast<const uint8_t*>(w0);
   a.w1 = static_cast<const uint8_t*>(w1);
@@ -533,7 +555,10 @@ hipError_t launch_tok_mm(const TokPlan& p, uint32_t quant, const void* w0, const
   a.tokens = tokens;
   a.groups = p.groups;
   a.q6s = reading;
-  const int64_t blocks = int64_t(p.nsplit) * ((p.tiles + 7) / 8) * p.groups * 8;
+  if (items) a.items = *items;
+  if (items && p.nsplit != 1) return hipErrorInvalidValue;
+  const int64_t blocks = items ? int64_t(p.groups + 7) / 8 * 8 * p.tiles
+                               : int64_t(p.nsplit) * ((p.tiles + 7) / 8) * p.groups * 8;
   if (blocks > (int64_t(1) << 31) - 1) return hipErrorInvalidValue;
   switch (quant) {
     case kQ4_K: launch_tok_f<TokQ4Q5<kQ4_K>>(p.tok, a, blocks, s); break;

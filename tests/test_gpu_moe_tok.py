@@ -1,0 +1,145 @@
+"""The MoE of many tokens over out-major expert stacks (moe_tok.hip) vs the
+oracle's out-major composition, at the sizes where it ends: every group size
+(8, 16, 32, 64 and 96 tokens of an expert), groups that run over, all tokens
+on the same experts, rows that are no multiple of the 128-row tiles, every
+type, both routing forms (above and at 16 tokens), the shared expert in the
+whole layer, gate and up in two Q6_K readings, and x at float alignment.
+
+Bars: conftest.check_parity's, a token at a time, as the two-token form's;
+twice the per-element one where the reference is the device's own few-token
+form, itself within one bar of the oracle.
+"""
+import numpy as np
+import pytest
+
+import strata_hip as H
+from conftest import STRICT_TOL, check_parity
+from strata_hip import synth as S
+from test_gpu_moe_om import OM, om_tensors, om_views, oracle_om, layer_om_tensors
+
+pytestmark = pytest.mark.gpu
+Q8_0, Q4_K, Q5_K, Q6_K, IQ4_XS = 8, 12, 13, 14, 23
+
+
+def moe_dev(quants, flags, mats, n_expert, n_embd, n_ff, logits, x, top_k, offset=0):
+    """offset: floats between x's start and a 256-byte boundary."""
+    import torch
+    n_tok = x.shape[0]
+    dev = [torch.from_numpy(np.ascontiguousarray(m)).cuda() for m in mats]
+    tl = torch.from_numpy(logits).cuda()
+    xb = torch.zeros(x.size + offset, device="cuda")
+    xb[offset:] = torch.from_numpy(x.reshape(-1)).cuda()
+    out = torch.full((n_tok, n_embd), float("nan"), device="cuda")
+    nb = H.moe_workspace_bytes(n_tok, top_k, n_expert, n_embd, n_ff, quants[0], quants[2])
+    ws = torch.full((nb,), 0xFF, dtype=torch.uint8, device="cuda")
+    H.moe_ffn_dev(*[(q, OM | f, t.data_ptr()) for q, f, t in zip(quants, flags, dev)], n_expert, n_embd, n_ff,
+                  tl.data_ptr(), n_tok, top_k, xb.data_ptr() + 4 * offset, out.data_ptr(), ws.data_ptr(), nb,
+                  torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("qg,qd,n_expert,n_embd,n_ff,top_k,n_tok", [
+    (Q4_K, Q6_K, 64, 512, 512, 4, 20),    # groups of 8
+    (Q5_K, Q4_K, 16, 512, 768, 6, 20),    # 16
+    (Q6_K, Q8_0, 8, 1024, 256, 3, 40),    # 32
+    (Q8_0, Q5_K, 4, 512, 768, 2, 60),     # 64
+    (Q4_K, Q6_K, 3, 768, 512, 2, 90),     # 96
+    (Q8_0, Q8_0, 24, 1088, 320, 4, 16),   # rows of 34 and 10 blocks, one routing launch
+    (IQ4_XS, Q4_K, 12, 256, 1024, 5, 17),
+    (Q6_K, Q6_K, 32, 768, 2304, 2, 15),
+])
+def test_moe_many_tokens(oracle, qg, qd, n_expert, n_embd, n_ff, top_k, n_tok):
+    print("[case] moe tokens", qg, qd, n_expert, n_embd, n_ff, top_k, n_tok, flush=True)
+    mats = om_tensors(n_expert, n_embd, n_ff, qg, qd, 60 + n_tok)
+    logits = S.router_logits(61 + n_tok, n_tok, n_expert)
+    x = S.normal_f32(62 + n_tok, n_tok * n_embd).reshape(n_tok, n_embd)
+    x[1] *= 50.0
+    x[3] = 0.0
+    got = moe_dev((qg, qg, qd), (0, 0, 0), mats, n_expert, n_embd, n_ff, logits, x, top_k)
+    want = oracle_om(oracle, qg, qd, n_expert, n_embd, n_ff, *mats, logits, x, top_k)
+    for t in range(n_tok):
+        check_parity(got[t], want[t], f"token {t}")
+    shifted = moe_dev((qg, qg, qd), (0, 0, 0), mats, n_expert, n_embd, n_ff, logits, x, top_k, offset=1)
+    assert np.array_equal(got, shifted)
+
+
+def test_moe_all_tokens_on_the_same_experts(oracle):
+    """Every token picks experts 0 and 1: groups of 16 run over six times."""
+    print("[case] moe tokens, two experts", flush=True)
+    n_expert, n_embd, n_ff, top_k, n_tok = 32, 512, 256, 2, 100
+    mats = om_tensors(n_expert, n_embd, n_ff, Q4_K, Q6_K, 70)
+    logits = np.zeros((n_tok, n_expert), np.float32)
+    x = S.normal_f32(71, n_tok * n_embd).reshape(n_tok, n_embd)
+    got = moe_dev((Q4_K, Q4_K, Q6_K), (0, 0, 0), mats, n_expert, n_embd, n_ff, logits, x, top_k)
+    want = oracle_om(oracle, Q4_K, Q6_K, n_expert, n_embd, n_ff, *mats, logits, x, top_k)
+    for t in range(n_tok):
+        check_parity(got[t], want[t], f"token {t}")
+
+
+@pytest.mark.parametrize("quant,flags", [(Q6_K, (H.FLAG_Q6K_SIGNED_SCALES, 0, H.FLAG_Q6K_SIGNED_SCALES)),
+                                         (Q6_K, (0, H.FLAG_Q6K_SIGNED_SCALES, 0)),
+                                         (IQ4_XS, (H.FLAG_IQ4XS_GGML,) * 3)])
+def test_moe_many_tokens_readings(quant, flags):
+    """The flagged readings (gate's and up's may differ for Q6_K), against
+    the same tokens four at a time (moe_om.hip)."""
+    print("[case] moe tokens, readings", quant, flags, flush=True)
+    n_expert, n_embd, n_ff, top_k, n_tok = 16, 512, 512, 4, 40
+    mats = om_tensors(n_expert, n_embd, n_ff, quant, quant, 80)
+    logits = S.router_logits(81, n_tok, n_expert)
+    x = S.normal_f32(82, n_tok * n_embd).reshape(n_tok, n_embd)
+    args = ((quant,) * 3, flags, mats, n_expert, n_embd, n_ff)
+    got = moe_dev(*args, logits, x, top_k)
+    for t in range(0, n_tok, 4):
+        want = moe_dev(*args, logits[t:t + 4], x[t:t + 4], top_k)
+        for i in range(4):
+            check_parity(got[t + i], want[i], f"token {t + i}", strict_tol=2 * STRICT_TOL)
+
+
+@pytest.mark.parametrize("n_sh,n_tok", [(256, 9), (768, 33), (512, 100)])
+def test_moe_layer_many_tokens(n_sh, n_tok):
+    """The whole layer (router and shared expert of many tokens in one set
+    of launches), against the same tokens four at a time; replayed from a
+    graph, eager calls between."""
+    import torch
+    print("[case] moe layer tokens", n_sh, n_tok, flush=True)
+    n_expert, n_embd, n_ff, top_k = 16, 768, 512, 6
+    q, t = layer_om_tensors(n_expert, n_embd, n_ff, n_sh, 90)
+    x = S.normal_f32(91, n_tok * n_embd).reshape(n_tok, n_embd)
+    bufs = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in t]
+    flags = [0, OM, OM, OM, 0, 0, 0, 0]
+    tensors = [(q[i], flags[i], bufs[i].data_ptr()) for i in range(8)]
+    tx = torch.from_numpy(x).cuda()
+    out = torch.full((n_tok, n_embd), float("nan"), device="cuda")
+    nb = H.moe_layer_workspace_bytes(n_tok, top_k, n_expert, n_embd, n_ff, n_sh, q)
+    ws = torch.full((nb,), 0xFF, dtype=torch.uint8, device="cuda")
+
+    def call(t0, n, o):
+        H.moe_layer_dev(tensors, n_expert, n_embd, n_ff, n_sh, n, top_k, tx.data_ptr() + 4 * t0 * n_embd, o.data_ptr(),
+                        ws.data_ptr(), nb, torch.cuda.current_stream().cuda_stream)
+
+    call(0, n_tok, out)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    few = torch.empty((4, n_embd), device="cuda")
+    for t0 in range(0, n_tok, 4):
+        n = min(4, n_tok - t0)
+        call(t0, n, few)
+        torch.cuda.synchronize()
+        for i in range(n):
+            check_parity(got[t0 + i], few[i].cpu().numpy(), f"token {t0 + i}", strict_tol=2 * STRICT_TOL)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        call(0, n_tok, out)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        call(0, n_tok, out)
+    for rep in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), got), rep
+        call(0, 4, few)
+        torch.cuda.synchronize()
