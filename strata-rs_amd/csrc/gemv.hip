@@ -24,6 +24,7 @@
 //     one; row sums are reduced across the wave with cross-lane shuffles.
 // Weight bytes are read exactly once per launch with 16-byte loads of the
 // block layout; nothing is dequantized to memory.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -128,6 +129,145 @@ __global__ void __launch_bounds__(512) gemv_kernel(const uint8_t* __restrict__ w
     win = nwn;
 #pragma unroll
     for (int i = 0; i < R; ++i) cur[i] = nxt[i];
+  }
+}
+
+// -------------------------------------------------- Q6_K, batches of 2..4 --
+// gemv_kernel reads Q6_K units of 52 bytes in a row from 64 addresses a load
+// (the load unit takes such a 16-byte load in 64 or more accesses) and
+// decodes them once per vector: the 151936 x 4096 head took 241 us for two
+// vectors and 253 for four, where the weights stream in about 91. Here a wave
+// takes two rows at a time, a window (64 units) of each in whole coalesced
+// pieces, the next ones in flight while it computes; the pieces pass through
+// the wave's LDS to the lanes' units, every weight becomes the f32 value
+// (q - 32) * sc once (exact: 14 bits), and both rows share each read of a
+// vector from LDS. Rows of whole 2048 columns (whole 16-byte pieces) on
+// 16-byte boundaries only. Bound by VALU issue (97% busy at four vectors: one fma a
+// weight and vector, about four instructions to form it): the head 241 -> 143
+// us for two vectors, 253 -> 203 for four, 421 -> 362 for eight; 4096 x 12288
+// 19.8 -> 17.5, 39 -> 34, 76 -> 67; 4096 x 4096 9.8 -> 8.0, 12.5 -> 10.3.
+// Error against 64 bits 1.9e-7 -> 1.1e-7 (no -32 * sum(x) to cancel).
+constexpr int kWinQ6 = 16 * 210;  // bytes of a window
+constexpr int kWinPieces = (kWinQ6 + 1023) / 1024;
+constexpr int kWinWaves = 12;  // a workgroup's at most
+
+// x as gemv_kernel's, without the sums
+__host__ __device__ inline int xw_stride(int cols) { return cols + cols / 16; }
+
+// the lane's unit of a window in LDS -> its 64 values (q - 32) * sc; returns d
+__device__ __forceinline__ float q6_unit(const uint8_t* win, int u, int q6_signed, f32x4 (&w)[16]) {
+  const int at = 210 * (u >> 2);
+  const uint32_t shift = uint32_t(at) & 3u, tp = uint32_t(u) & 1u;
+  const int h = (u >> 1) & 1;
+  const uint32_t* base = reinterpret_cast<const uint32_t*>(win + at - int(shift));
+  uint32_t l[17], hb[9];
+#pragma unroll
+  for (int k = 0; k < 17; ++k) l[k] = base[16 * h + k];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) hb[k] = base[32 + 8 * h + k];
+  const uint32_t* sp = base + 48 + 2 * h + int(tp);
+  const uint32_t scw = __builtin_amdgcn_alignbyte(sp[1], sp[0], shift);
+  float sc[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    sc[j] = q6_signed ? float(int8_t(scw >> (8 * j))) : float((scw >> (8 * j)) & 0xFFu);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    uint32_t a, b;
+    q6_code_words(l[k], l[k + 1], l[8 + k], l[9 + k], hb[k], hb[k + 1], shift, tp, a, b);
+    const float s0 = sc[k >> 2], s1 = sc[2 + (k >> 2)], m0 = -32.f * s0, m1 = -32.f * s1;
+    w[k] = f32x4{__builtin_fmaf(ubyte<0>(a), s0, m0), __builtin_fmaf(ubyte<1>(a), s0, m0),
+                 __builtin_fmaf(ubyte<2>(a), s0, m0), __builtin_fmaf(ubyte<3>(a), s0, m0)};
+    w[8 + k] = f32x4{__builtin_fmaf(ubyte<0>(b), s1, m1), __builtin_fmaf(ubyte<1>(b), s1, m1),
+                     __builtin_fmaf(ubyte<2>(b), s1, m1), __builtin_fmaf(ubyte<3>(b), s1, m1)};
+  }
+  return h2f(*reinterpret_cast<const uint16_t*>(win + at + 208));
+}
+
+template <int NB>
+__global__ void __launch_bounds__(64 * kWinWaves)
+    gemv_q6win_kernel(const uint8_t* __restrict__ w, int rows, int cols, int64_t row_bytes, const float* __restrict__ x,
+                      float* __restrict__ y, int q6_signed) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int xs = xw_stride(cols);
+  const int units = cols >> 6, nwin = (units + 63) >> 6;
+  const int wpg = blockDim.x >> 6;
+  const int n_rg = (rows + 1) >> 1, stride = gridDim.x * wpg;
+  int rg = blockIdx.x * wpg + wave, win = 0;
+  // a window's pieces of both rows (past the window: its last piece again)
+  u32x4 p[2][kWinPieces];
+  auto issue = [&](int g, int wn) {
+    const int last = min(kWinQ6, int(row_bytes) - wn * kWinQ6) - 16;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint8_t* src = w + int64_t(min(2 * g + i, rows - 1)) * row_bytes + wn * kWinQ6;
+#pragma unroll
+      for (int k = 0; k < kWinPieces; ++k) p[i][k] = ld16(src + min(16 * lane + 1024 * k, last));
+    }
+  };
+  if (rg < n_rg) issue(rg, 0);
+  for (int i = tid; i < NB * (cols >> 2); i += blockDim.x) {
+    const int b = i / (cols >> 2), c = 4 * (i - b * (cols >> 2));
+    *reinterpret_cast<f32x4*>(lds + b * xs + c + 4 * (c >> 6)) =
+        *reinterpret_cast<const f32x4*>(x + int64_t(b) * cols + c);
+  }
+  __syncthreads();
+  uint8_t* buf = reinterpret_cast<uint8_t*>(lds + NB * xs) + wave * (2 * kWinQ6);
+  float acc[2][NB];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[i][b] = 0.f;
+  while (rg < n_rg) {
+    // into LDS (a wave's LDS operations run in order: its reads below see
+    // every lane's pieces, its next writes come after them)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int k = 0; k < kWinPieces; ++k) {
+        const int off = 16 * lane + 1024 * k;
+        if (off < kWinQ6) *reinterpret_cast<u32x4*>(buf + i * kWinQ6 + off) = p[i][k];
+      }
+    int nrg = rg, nwn = win + 1;
+    if (nwn == nwin) {
+      nwn = 0;
+      nrg = rg + stride;
+    }
+    if (nrg < n_rg) issue(nrg, nwn);
+    const int u = min(64 * win + lane, units - 1);  // lanes past the row: the last unit, not added
+    const bool on = 64 * win + lane < units;
+    f32x4 w0[16], w1[16];
+    const float d0 = q6_unit(buf, u & 63, q6_signed, w0);
+    const float d1 = q6_unit(buf + kWinQ6, u & 63, q6_signed, w1);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const f32x4* xv = reinterpret_cast<const f32x4*>(lds + b * xs + 68 * u);
+      f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const f32x4 v = xv[k];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          s0[j] = __builtin_fmaf(w0[k][j], v[j], s0[j]);
+          s1[j] = __builtin_fmaf(w1[k][j], v[j], s1[j]);
+        }
+      }
+      acc[0][b] += on ? d0 * ((s0.x + s0.y) + (s0.z + s0.w)) : 0.f;
+      acc[1][b] += on ? d1 * ((s1.x + s1.y) + (s1.z + s1.w)) : 0.f;
+    }
+    if (win == nwin - 1) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const float t = wave_sum_dpp(acc[i][b]);
+          if (lane == 63 && 2 * rg + i < rows) y[int64_t(b) * rows + 2 * rg + i] = t;
+          acc[i][b] = 0.f;
+        }
+    }
+    rg = nrg;
+    win = nwn;
   }
 }
 
@@ -818,6 +958,33 @@ static hipError_t launch_nb(int nb, const uint8_t* w, int rows, int cols, int64_
   }
 }
 
+// Vectors per launch of gemv_q6win_kernel (as even as they go), 0: a shape it
+// does not take.
+static size_t q6win_lds(int cols, int nb, int waves) {
+  return size_t(nb) * xw_stride(cols) * sizeof(float) + size_t(waves) * 2 * kWinQ6;
+}
+static int q6win_batch(const uint8_t* w, int cols, int batch) {
+  if (batch < 2 || cols % 2048 != 0 || (reinterpret_cast<uintptr_t>(w) & 15u)) return 0;
+  int most = 4;
+  while (most >= 2 && q6win_lds(cols, most, 8) > kMaxLds) --most;
+  if (most < 2) return 0;
+  const int n = (batch + most - 1) / most, per = (batch + n - 1) / n;
+  // (the last launch takes what is left, at least two)
+  return batch - (n - 1) * per >= 2 || n == 1 ? per : 0;
+}
+template <int NB>
+static void launch_q6win(const uint8_t* w, int rows, int cols, int64_t rb, const float* x, float* y, int q6s,
+                         hipStream_t s) {
+  // 12 waves where LDS holds their windows and each has two items at least
+  // (151936 x 4096, 4 vectors: 8 waves 219 us, 12 203; 4096 x 4096: 10.3, 11.2)
+  const int n_rg = (rows + 1) / 2;
+  const int wpg = q6win_lds(cols, NB, kWinWaves) <= kMaxLds && n_rg >= 2 * kWinWaves * cu_count() ? kWinWaves : 8;
+  const size_t lds = q6win_lds(cols, NB, wpg);
+  const int most = cu_count() * (2 * lds <= kMaxLds ? 2 : 1), blocks = std::min(most, (n_rg + wpg - 1) / wpg);
+  hipLaunchKernelGGL(gemv_q6win_kernel<NB>, dim3(unsigned(blocks)), dim3(unsigned(64 * wpg)), lds, s, w, rows, cols, rb, x, y,
+                     q6s);
+}
+
 // Batched Q4_K / Q5_K rows convert their activations once per call into the
 // workspace (each workgroup then copies its window rather than converting
 // it), and rows wider than one window run split-K over the windows.
@@ -851,6 +1018,20 @@ hipError_t launch_gemv(uint32_t quant, const void* wv, int64_t rows, int64_t col
     return hipErrorInvalidValue;
   if (batch >= 2 && gemv_mfma_ok(quant, rows, cols, batch))
     return launch_gemv_mfma(quant, w, rows, cols, x, y, batch, cu_count(), stream, ws);
+  if (const int per = quant == kQ6_K ? q6win_batch(w, int(cols), batch) : 0) {
+    for (int b0 = 0; b0 < batch; b0 += per) {
+      const float* xb = x + int64_t(b0) * cols;
+      float* yb = y + int64_t(b0) * rows;
+      switch (std::min(per, batch - b0)) {
+        case 2: launch_q6win<2>(w, int(rows), int(cols), row_bytes, xb, yb, q6_signed, stream); break;
+        case 3: launch_q6win<3>(w, int(rows), int(cols), row_bytes, xb, yb, q6_signed, stream); break;
+        default: launch_q6win<4>(w, int(rows), int(cols), row_bytes, xb, yb, q6_signed, stream);
+      }
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
   // batch 1: 16 waves per CU for tall matrices whose rows are a single
   // 4096-column window (more waves hide more latency, and each still has
   // rows to stream); 8 otherwise (fewer workgroups stage x, and multi-window
