@@ -12,8 +12,8 @@
 // the tokens, gate and up in one launch, silu(g) * u converted, down, and the
 // sum of down's shares with the residual (six launches for any number of
 // tokens; the weights are read once per 96 tokens instead of once per 8:
-// Q4_K gate and up, Q6_K down at 4096 / 12288, 9 tokens 139 -> 98 us, 24
-// tokens 327 -> 65, 77 tokens 1015 -> 118, 512 tokens 6631 -> 527). Otherwise
+// Q4_K gate and up, Q6_K down at 4096 / 12288, 9 tokens 139 -> 60 us, 24
+// tokens 327 -> 63, 77 tokens 1015 -> 118, 512 tokens 6631 -> 527). Otherwise
 // each step is its own launch (matvecs 8 tokens at a time; at 2 tokens that
 // is still the faster form, 55 against 57 us).
 #include <algorithm>
@@ -39,10 +39,10 @@ struct FfnTok {
   TokPlan gu, dn;
   size_t o_part, bytes;
 };
-static FfnTok ffn_tok_plan(int64_t n_tok, int64_t n_embd, int64_t n_ff, int max_split) {
+static FfnTok ffn_tok_plan(int64_t n_tok, int64_t n_embd, int64_t n_ff, int gu_split, int dn_split) {
   FfnTok p{};
-  p.gu = tok_plan(n_ff, 2, n_embd, int(n_tok), cu_count(), max_split);
-  p.dn = tok_plan(n_embd, 1, n_ff, int(n_tok), cu_count(), max_split);
+  p.gu = tok_plan(n_ff, 2, n_embd, int(n_tok), cu_count(), gu_split);
+  p.dn = tok_plan(n_embd, 1, n_ff, int(n_tok), cu_count(), dn_split);
   const size_t T = size_t(n_tok) * sizeof(float);
   p.o_part = align256(std::max(tok_image_bytes(p.gu), tok_image_bytes(p.dn)));
   p.bytes = p.o_part + align256(std::max({T * n_embd, T * 2 * n_ff * p.gu.nsplit, T * n_embd * p.dn.nsplit}));
@@ -52,11 +52,13 @@ constexpr int kFfnMaxSplit = 8;
 
 // Small calls keep the size of the step-by-step form, which the fixed
 // scratch of the allocation-free entry point holds; the many-token form then
-// takes as many shares as fit. Larger ones have room for all it asks for.
+// takes as many shares as fit, of each product by itself (17 tokens at 4096 /
+// 12288: one share of gate and up fills what is left, but eight of down do not;
+// with one of each the call took 190 us, so 78). Larger ones have room for all it asks for.
 size_t ffn_workspace_bytes(int64_t n_tok, int64_t n_embd, int64_t n_ff) {
   const size_t steps = ffn_step_bytes(n_tok, n_embd, n_ff);
   if (n_tok <= 8 || n_tok > kFfnMaxTokTokens) return steps;
-  const size_t tok = ffn_tok_plan(n_tok, n_embd, n_ff, kFfnMaxSplit).bytes;
+  const size_t tok = ffn_tok_plan(n_tok, n_embd, n_ff, kFfnMaxSplit, kFfnMaxSplit).bytes;
   return std::max(steps, steps <= kFfnFixedScratch ? std::min(tok, kFfnFixedScratch) : tok);
 }
 
@@ -90,9 +92,11 @@ hipError_t launch_ffn(uint32_t q_gate, uint32_t q_up, uint32_t q_down, const voi
   if (n_tok > 8 && n_tok <= kFfnMaxTokTokens && q_gate == q_up && q6g == q6u && tok_ok(q_gate, n_ff, n_embd) &&
       tok_ok(q_down, n_embd, n_ff)) {
     const size_t room = ffn_workspace_bytes(n_tok, n_embd, n_ff);
-    int split = kFfnMaxSplit;
-    FfnTok p = ffn_tok_plan(n_tok, n_embd, n_ff, split);
-    while (p.bytes > room && split > 1) p = ffn_tok_plan(n_tok, n_embd, n_ff, --split);
+    int gu_split = kFfnMaxSplit, dn_split = kFfnMaxSplit;
+    FfnTok p = ffn_tok_plan(n_tok, n_embd, n_ff, gu_split, 1);
+    while (p.bytes > room && gu_split > 1) p = ffn_tok_plan(n_tok, n_embd, n_ff, --gu_split, 1);
+    p = ffn_tok_plan(n_tok, n_embd, n_ff, gu_split, dn_split);
+    while (p.bytes > room && dn_split > 1) p = ffn_tok_plan(n_tok, n_embd, n_ff, gu_split, --dn_split);
     if (p.bytes <= room) {
       float* part = reinterpret_cast<float*>(ws + p.o_part);
       const int64_t nx = int64_t(T) * n_embd, ng = int64_t(T) * 2 * n_ff;
