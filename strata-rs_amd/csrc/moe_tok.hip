@@ -28,18 +28,21 @@ static TokPlan moe_tok_plan(const MoePlan& p, int rows, int mats, int cols) {
 }
 
 // Pairs per work item, by an expert's average (a group past it reads the
-// weights again, from L2 at best; the smaller fragments cost less LDS), or 0:
+// weights again, from L2 at best; fragments of 16 leave the LDS for one
+// workgroup a CU beside the weights: 96 tokens of 128 experts, average 6, take
+// 169 us in groups of 8, 217 of 16, 191 of 32; 256 tokens, average 16, 299, 302
+// and 214), or 0:
 // moe_om.hip's launches, three fewer and one pass over the weights per two
 // pairs, stay the faster form for few pairs of small experts. Both measured,
-// Q4_K / Q6_K 128 x 2048 x 768 top-8: 4 tokens 59 against 60 us, 6 84 / 75, 16
-// 176 / 109, 96 640 / 209, 256 1465 / 238; Q5_K / Q8_0 32 x 1280 x 512 top-2:
-// 8 tokens 29 / 35, 16 39 / 38, 64 81 / 46, 256 242 / 53.
+// Q4_K / Q6_K 128 x 2048 x 768 top-8: 4 tokens 59 against 60 us, 8 99 / 75, 16
+// 176 / 97, 96 640 / 169, 256 1465 / 203; Q5_K / Q8_0 32 x 1280 x 512 top-2:
+// 8 tokens 29 / 35, 16 39 / 36, 64 81 / 42, 256 242 / 53.
 int moe_tok_group(const MoePlan& p, uint32_t qa, uint32_t qb) {
   if (!tok_ok(qa, p.n_ff, p.n_embd) || !tok_ok(qb, p.n_embd, p.n_ff)) return 0;
   const int64_t pairs = int64_t(p.n_tok) * p.top_k, work = pairs * p.n_embd * p.n_ff;
   if (p.n_tok <= 4 || work < (p.n_tok >= 16 ? 20000000 : 50000000)) return 0;
   const int64_t avg = (pairs + p.s_max - 1) / p.s_max;
-  return avg <= 4 ? 8 : avg <= 8 ? 16 : avg <= 24 ? 32 : avg <= 48 ? 64 : 96;
+  return avg <= 8 ? 8 : avg <= 32 ? 32 : avg <= 64 ? 64 : 96;
 }
 
 size_t moe_tok_image_bytes(const MoePlan& p) {

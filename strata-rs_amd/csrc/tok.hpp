@@ -93,6 +93,8 @@ __device__ __forceinline__ void tok_signed4(uint32_t w, f16x2_t& a, f16x2_t& b) 
 // sub-block scales of the k steps (kSub 1) or sub-blocks (kSub 2). kSub 0:
 // the scales are in the weights. `left`: Q8_0 blocks from the super-block's
 // first to the row's last.
+// take_lds<g>: take<g> from the row's bytes in LDS (kPieces 16-byte pieces
+// from the dword at or below the super-block, `sh` bytes below it).
 // kPerm 0: step i of lane half h is columns 16 h + 8 i + [0, 8) of the
 // sub-block; 1: columns 16 i + 8 h + [0, 8).
 template <int Q>
@@ -120,6 +122,17 @@ struct TokQ4Q5 {  // Q4_K, Q5_K
     if constexpr (G == 0) {
       s.h = r.h;
       if constexpr (Q == kQ5_K) s.qh = r.qh;
+      s.sc03 = s.h.y & 0x3F3F3F3Fu;
+      s.sc47 = (s.h.w & 0x0F0F0F0Fu) | ((s.h.y >> 2) & 0x30303030u);
+    }
+  }
+  static constexpr int kPieces = kSbBytes / 16;
+  template <int G>
+  __device__ static __forceinline__ void take_lds(const uint8_t* row, uint32_t, uint32_t, int half, Sb& s) {
+    s.q = *reinterpret_cast<const u32x4*>(row + (Q == kQ5_K ? 48 : 16) + 32 * G + 16 * half);
+    if constexpr (G == 0) {
+      s.h = *reinterpret_cast<const u32x4*>(row);
+      if constexpr (Q == kQ5_K) s.qh = *reinterpret_cast<const u32x4*>(row + 16 + 16 * half);
       s.sc03 = s.h.y & 0x3F3F3F3Fu;
       s.sc47 = (s.h.w & 0x0F0F0F0Fu) | ((s.h.y >> 2) & 0x30303030u);
     }
@@ -213,6 +226,23 @@ struct TokQ6 {
     const auto b = __builtin_amdgcn_permlane32_swap(w.y, w.w, false, false);
     return u32x4{a[0], b[0], a[1], b[1]};
   }
+  static constexpr int kPieces = 13;  // 208 bytes; the last dword is the row's `tail`
+  __device__ static __forceinline__ u32x4 lds16(const uint8_t* p, uint32_t sh) {
+    return win16({*reinterpret_cast<const u32x4*>(p), *reinterpret_cast<const uint32_t*>(p + 16)}, sh);
+  }
+  template <int G>
+  __device__ static __forceinline__ void take_lds(const uint8_t* row, uint32_t sh, uint32_t tail, int half, Sb& s) {
+    if constexpr (G == 0) {
+      s.sc = win16({*reinterpret_cast<const u32x4*>(row + 192), tail}, sh);
+      s.d = (tail >> (8 * sh)) & 0xFFFFu;
+    }
+    if constexpr ((G & 1) == 0) {
+      constexpr int H = G >> 1;
+      s.qh = halves(lds16(row + 128 + 32 * H + 16 * half, sh));
+      s.ql[0] = halves(lds16(row + 64 * H + 16 * half, sh));
+      s.ql[1] = halves(lds16(row + 64 * H + 32 + 16 * half, sh));
+    }
+  }
   __device__ static __forceinline__ float d(const Sb& s) { return h2f(s.d); }
   template <int G>
   __device__ static __forceinline__ void take(const Raw& r, Sb& s) {
@@ -293,6 +323,18 @@ struct TokQ8 {
     s.q[1] = r.q[2 * G + 1];
     s.d[0] = r.d[2 * G];
     s.d[1] = r.d[2 * G + 1];
+  }
+  static constexpr int kPieces = 17;  // rows of whole super-blocks
+  template <int G>
+  __device__ static __forceinline__ void take_lds(const uint8_t* row, uint32_t, uint32_t, int half, Sb& s) {
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      constexpr int J = 2 * G;
+      const uint32_t* p = reinterpret_cast<const uint32_t*>(row + ((34 * (J + jj) + 2) & ~3) + 16 * half);
+      const uint32_t sh = (34 * (J + jj) + 2) & 2;
+      s.q[jj] = win16({u32x4{p[0], p[1], p[2], p[3]}, sh ? p[4] : 0u}, sh);
+      s.d[jj] = *reinterpret_cast<const uint16_t*>(row + 34 * (J + jj));
+    }
   }
   __device__ static __forceinline__ float d(const Sb&) { return 1.f; }
   template <int G>

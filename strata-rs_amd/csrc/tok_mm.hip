@@ -180,7 +180,87 @@ struct TokMm {
   TokItems items;
 };
 
-template <class F, int TOK>
+struct TokNone {};
+template <class F>
+constexpr bool tok_lds_format() {
+  return !std::is_same<F, TokIQ4<true>>::value && !std::is_same<F, TokIQ4<false>>::value;
+}
+// A wave's 32 rows of a super-block on their way through its LDS: load()
+// requests them in whole 16-byte pieces, row after row (adjacent lanes read
+// adjacent bytes), store() writes the pieces that came to the wave's slot, in
+// the order they were read, and the lanes take their rows from there. Loads
+// straight to the lanes (32 rows x 32 bytes each) cost an access or two per
+// lane: Q6_K down of 96 tokens x 8 of 128 experts took 36 M accesses for 165
+// MB, and the load unit bound it. Routed FFN, 128 x 2048 x 768 Q4_K / Q6_K: 16
+// tokens 111 -> 98 us, 64 189 -> 155, 96 204 -> 169, 256 231 -> 214; dense FFN
+// 2048 / 6144 Q5_K / Q8_0, 12 tokens 43 -> 34.
+template <class F, bool CO>
+struct TokWave {
+  static constexpr int kN = (32 * F::kPieces + 63) / 64, kLds = kN * 1024;
+  static constexpr bool kTail = F::kSbBytes % 16 != 0;  // a dword past the pieces, rows off the dword grid
+  uint8_t* slot;
+  const uint8_t* base;  // a dword boundary at or below the wave's first row's share
+  uint32_t off[kN];     // of the lane's pieces (their rows') from it
+  uint32_t toff;        // of the lane's row
+  u32x4 v[kN];
+  uint32_t t;
+  uint32_t sh, tail;  // of the super-block in the slot: the lane's row
+  __device__ __forceinline__ TokWave(const uint8_t* w, int row0, int rows, int64_t rb, int sb0, uint8_t* l, int wave,
+                                     int lane) {
+    slot = l + wave * kLds;
+    const uint8_t* p = w + int64_t(min(row0, rows - 1)) * rb + int64_t(sb0) * F::kSbBytes;
+    const uint32_t b = uint32_t(reinterpret_cast<uintptr_t>(p)) & 3u;
+    base = p - b;
+    const int most = max(rows - 1 - row0, 0);  // rows past the matrix: its last
+#pragma unroll
+    for (int k = 0; k < kN; ++k) {
+      const int q = min(lane + 64 * k, 32 * F::kPieces - 1), r = q / F::kPieces;
+      off[k] = b + uint32_t(min(r, most)) * uint32_t(rb) + (kTail ? 0 : 16 * (q - r * F::kPieces));
+    }
+    toff = b + uint32_t(min(lane & 31, most)) * uint32_t(rb);
+  }
+  __device__ __forceinline__ void load(int s) {
+    const uint8_t* p = base + int64_t(s) * (kTail ? 0 : F::kSbBytes);
+    const uint32_t add = kTail ? uint32_t(s) * F::kSbBytes : 0;
+#pragma unroll
+    for (int k = 0; k < kN; ++k) {
+      typedef uint32_t u32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
+      uint32_t o = off[k];
+      if constexpr (kTail) {  // the dword at or below the row's super-block, then the piece
+        const int q = min(int(threadIdx.x & 63) + 64 * k, 32 * F::kPieces - 1);
+        o = ((o + add) & ~3u) + 16 * (q % F::kPieces);
+      }
+      const u32x4a4 x = *reinterpret_cast<const u32x4a4*>(p + o);
+      v[k] = u32x4{x.x, x.y, x.z, x.w};
+    }
+    if constexpr (kTail) t = *reinterpret_cast<const uint32_t*>(p + ((toff + add) & ~3u) + 16 * F::kPieces);
+  }
+  __device__ __forceinline__ void store(int s) {
+    const int lane = threadIdx.x & 63;
+    // (a wave's LDS operations run in order: its reads below see every
+    // lane's pieces, its next writes come after them)
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int k = 0; k < kN; ++k) *reinterpret_cast<u32x4*>(slot + 1024 * k + 16 * lane) = v[k];
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+    sh = kTail ? (toff + uint32_t(s) * F::kSbBytes) & 3u : 0;
+    tail = t;
+  }
+  __device__ __forceinline__ const uint8_t* row(int r32) const { return slot + r32 * (16 * F::kPieces); }
+};
+template <class F>
+struct TokWave<F, false> {
+  uint32_t sh, tail;
+  __device__ __forceinline__ TokWave(const uint8_t*, int, int, int64_t, int, uint8_t*, int, int) {}
+  __device__ __forceinline__ void load(int) {}
+  __device__ __forceinline__ void store(int) {}
+  __device__ __forceinline__ const uint8_t* row(int) const { return nullptr; }
+};
+
+// CO: the wave's weights by way of its own LDS (TokWave) instead of one
+// 16-byte load a lane from 32 rows at a time.
+template <class F, int TOK, bool CO>
 __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
   using S = TokShape<TOK>;
   constexpr int NT = S::kTiles;
@@ -225,7 +305,10 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
   const uint8_t* img = a.img + (int64_t(group) * a.nsb + sb0) * S::kSb;
   const int blk0 = a.nblk - 8 * sb0;  // blocks from this share's first
 
-  typename F::Raw raw0, raw1;  // even and odd super-blocks: no copies between them
+  using Raw = typename std::conditional<CO, TokNone, typename F::Raw>::type;
+  Raw raw0, raw1;  // even and odd super-blocks: no copies between them
+  TokWave<F, CO> wv((mat ? a.w1 : a.w0) + we, row0, a.rows, a.rb, sb0,
+                    lds + (S::kPacked ? 3 * S::kSb : 3 * S::kGroup + S::kSums + 1024), wave, lane);
   typename F::Sb sb;
   f32x16_t y[NT];
 #pragma unroll
@@ -306,9 +389,12 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
       }
     }
   };
-  auto load_sb = [&](int s, auto G, typename F::Raw& raw) {
+  auto load_sb = [&](int s, auto G, Raw& raw) {
     const int sc = min(s, n - 1);
-    F::template load<decltype(G)::value>(wr + int64_t(sc) * F::kSbBytes, half, raw, blk0 - 8 * sc);
+    if constexpr (!CO)
+      F::template load<decltype(G)::value>(wr + int64_t(sc) * F::kSbBytes, half, raw, blk0 - 8 * sc);
+    else if constexpr (decltype(G)::value == 0)
+      wv.load(sc);
     asm volatile("" ::: "memory");  // the loads stay here, a super-block ahead of their use
   };
   using std::integral_constant;
@@ -317,6 +403,13 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
   const integral_constant<int, 2> g2;
   const integral_constant<int, 3> g3;
 
+  auto take = [&](auto G, const Raw& cur) {
+    constexpr int g = decltype(G)::value;
+    if constexpr (CO)
+      F::template take_lds<g>(wv.row(r32), wv.sh, wv.tail, half, sb);
+    else
+      F::template take<g>(cur, sb);
+  };
   if constexpr (S::kPacked) {
     // stage = super-block: kCopies copies a wave (past the image: its last
     // KiB again, the same bytes to the same place)
@@ -338,7 +431,7 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
     stage(1, 1);
     wait_vmem<kCopies>();
     int slot = 0;
-    auto super_block = [&](int s, typename F::Raw& cur, typename F::Raw& next) {
+    auto super_block = [&](int s, Raw& cur, Raw& next) {
       // weights of s and stage s have landed when no more than the newest
       // kCopies operations, stage s + 1's copies, are outstanding. The next
       // weights go out ahead of the next copies: a wait for them with copies
@@ -346,6 +439,7 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
       // memory operation past a pending LDS copy)
       wait_vmem<kCopies>();
       lds_barrier();
+      if constexpr (CO) wv.store(s);
       load_sb(s + 1, g0, next);
       load_sb(s + 1, g1, next);
       load_sb(s + 1, g2, next);
@@ -354,13 +448,13 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
       const uint8_t* A = lds + slot * S::kSb;
       const int left = blk0 - 8 * s;
       f32x16_t acc[NT] = {};
-      F::template take<0>(cur, sb);
+      take(g0, cur);
       group_mma(g0, A, acc, left);
-      F::template take<1>(cur, sb);
+      take(g1, cur);
       group_mma(g1, A + S::kGroup, acc, left);
-      F::template take<2>(cur, sb);
+      take(g2, cur);
       group_mma(g2, A + 2 * S::kGroup, acc, left);
-      F::template take<3>(cur, sb);
+      take(g3, cur);
       group_mma(g3, A + 3 * S::kGroup, acc, left);
       finish_sb(A + 4 * S::kGroup, acc);
       slot = slot == 2 ? 0 : slot + 1;
@@ -392,7 +486,7 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
     stage(1, 1);
     wait_vmem<kCopies>();
     int slot = 0;
-    auto super_block = [&](int s, typename F::Raw& cur, typename F::Raw& next) {
+    auto super_block = [&](int s, Raw& cur, Raw& next) {
       f32x16_t acc[NT] = {};
       const int left = blk0 - 8 * s;
       auto step = [&](auto G) {
@@ -402,13 +496,17 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
         // next copies overwrite
         wait_vmem<kCopies>();
         lds_barrier();
+        if constexpr (CO && g == 0) {
+          wv.store(s);
+          load_sb(s + 1, G, next);
+        }
         if constexpr (g == 0) {
           const int q = min(wave, NT);  // NT fragments and one KiB of 2^-k
           copy16_to_lds(img + int64_t(s) * S::kSb + 4 * S::kGroup + q * 1024 + 16 * lane, tail + q * 1024);
         }
         stage(4 * s + g + 2, slot == 0 ? 2 : slot - 1);
-        F::template take<g>(cur, sb);
-        load_sb(s + 1, G, next);
+        take(G, cur);
+        if constexpr (!CO) load_sb(s + 1, G, next);
         group_mma(G, lds + slot * S::kGroup, acc, left);
         slot = slot == 2 ? 0 : slot + 1;
       };
@@ -522,7 +620,19 @@ template <class F, int TOK>
 static void launch_tok(const TokMm& a, int64_t blocks, hipStream_t s) {
   using S = TokShape<TOK>;
   const size_t lds = S::kPacked ? 3 * size_t(S::kSb) : 3 * size_t(S::kGroup) + S::kSums + 1024;
-  hipLaunchKernelGGL((tok_mm_kernel<F, TOK>), dim3(unsigned(blocks)), dim3(kTokThreads), lds, s, a);
+  // weights by way of LDS: up to 32 tokens (with more a super-block's MFMAs
+  // cover its loads, and the LDS costs a workgroup on the CU: 77 tokens of the
+  // dense FFN 116 us direct, 127 by way of LDS), pieces on the dword grid
+  // (Q6_K: realigned as they are read), rows of whole super-blocks
+  if constexpr (tok_lds_format<F>() && TOK <= 32) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(a.w0) | reinterpret_cast<uintptr_t>(a.w1) | uintptr_t(a.items.stride);
+    if (F::kSbBytes % 4 != 0 || ((at & 3u) == 0 && a.rb % F::kSbBytes == 0)) {
+      hipLaunchKernelGGL((tok_mm_kernel<F, TOK, true>), dim3(unsigned(blocks)), dim3(kTokThreads),
+                         (lds + 4 * TokWave<F, true>::kLds), s, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((tok_mm_kernel<F, TOK, false>), dim3(unsigned(blocks)), dim3(kTokThreads), lds, s, a);
 }
 template <class F>
 static void launch_tok_f(int tok, const TokMm& a, int64_t blocks, hipStream_t s) {
