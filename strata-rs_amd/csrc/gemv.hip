@@ -453,21 +453,19 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
 }
 constexpr int kLimbMaxRowsOneWin = 64;  // row groups a wave may take when rows are one window
 
+// The work of workgroup `block` of `blocks`.
 template <class F, int R, int MAXQ, int MODE = 0, int NPRE = 1, bool SPREAD = false>
-__global__ void __launch_bounds__(512) gemv_limb_kernel(const uint8_t* __restrict__ w, int rows,
-                                                        int cols, int64_t row_bytes,
-                                                        const float* __restrict__ x,
-                                                        float* y, int per, int flags,
-                                                        const uint8_t* __restrict__ w2, int rows1,
-                                                        const float* __restrict__ xu,
-                                                        const float* xres) {  // xres may be y (in place)
+__device__ __forceinline__ void limb_rows(const uint8_t* __restrict__ w, int rows, int cols, int64_t row_bytes,
+                                          const float* __restrict__ x, float* y, int per, int flags,
+                                          const uint8_t* __restrict__ w2, int rows1, const float* __restrict__ xu,
+                                          const float* xres, int block, int blocks) {  // xres may be y (in place)
   extern __shared__ __attribute__((aligned(16))) uint8_t lds8[];
   constexpr bool kLow = F::kQuant == kQ8_0 || F::kQuant == kIQ4_XS;  // signed codes: the low-limb sums
   // 23-bit limbs for every step of the silu(g) * u chain: the gate / up
   // inputs whose sums form it and the inputs formed from it
   constexpr bool kFine = (MODE & (kLimbTwoMat | kLimbPairSilu | kLimbSiluX | kLimbResid | kLimbFine)) != 0;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (tid >> 6));
+  const int wave = __builtin_amdgcn_readfirstlane(block * int(blockDim.x >> 6) + (tid >> 6));
   const int units = cols >> 6;
   const int nwin = (units + 63) >> 6;
   const int n_rg = (rows + R - 1) / R;
@@ -477,7 +475,7 @@ __global__ void __launch_bounds__(512) gemv_limb_kernel(const uint8_t* __restric
   // stretch of the matrix at a time (the 151936-row Q6_K head: 111 -> 104
   // us). No division here: it would delay the first weight loads.
   static_assert(!SPREAD || NPRE == 1, "spread rows are single-window rows");
-  const int W = int(gridDim.x) * int(blockDim.x >> 6);
+  const int W = blocks * int(blockDim.x >> 6);
   const int gstep = SPREAD ? W : 1;
   const int rg0 = SPREAD ? wave : wave * per;
   const int my = SPREAD ? max(0, per - (wave + (per - 1) * W >= n_rg ? 1 : 0)) : max(0, min(per, n_rg - rg0));
@@ -648,6 +646,15 @@ __global__ void __launch_bounds__(512) gemv_limb_kernel(const uint8_t* __restric
   }
 }
 
+template <class F, int R, int MAXQ, int MODE = 0, int NPRE = 1, bool SPREAD = false>
+__global__ void __launch_bounds__(512) gemv_limb_kernel(const uint8_t* __restrict__ w, int rows, int cols,
+                                                        int64_t row_bytes, const float* __restrict__ x, float* y,
+                                                        int per, int flags, const uint8_t* __restrict__ w2, int rows1,
+                                                        const float* __restrict__ xu, const float* xres) {
+  limb_rows<F, R, MAXQ, MODE, NPRE, SPREAD>(w, rows, cols, row_bytes, x, y, per, flags, w2, rows1, xu, xres,
+                                            int(blockIdx.x), int(gridDim.x));
+}
+
 // ------------------------------------------------------- F32 / F16 / BF16 --
 // Plain-float rows (quant.rs ids 0, 1, 30: the router and shared-expert gate
 // tensors real files carry). As ops::gemv (ops.rs:14-28) every product
@@ -724,6 +731,63 @@ __global__ void __launch_bounds__(kPlainThreads) gemv_plain_kernel(const uint8_t
       y2[int64_t(b0 + tid) * rows2 + r] = float(v);
     else
       y[int64_t(b0 + tid) * rows + r] = float(v);
+  }
+}
+
+// One token's router row, gate-input row and shared-expert gate / up rows in
+// one launch (all read x alone): workgroups [0, n_limb) are kLimbPairSilu's,
+// the rest take two plain rows each, 256 threads a row, summed as
+// gemv_plain_kernel sums them. Apart they are two launches of 3.2 and 4.2 us
+// at 128 x 2048 and 2 x 768 x 2048, neither of which fills the chip.
+struct MoeFront {
+  const uint8_t *w, *w2;  // router (`rows` rows against bf16(x)), gate input (one row against x)
+  int rows;
+  int64_t rb;
+  float *y, *y2;
+  const uint8_t *gate, *up;  // the shared expert's: n_ff rows each
+  int n_ff;
+  int64_t rb_sh;
+  float* h;  // silu(g) * u
+  int per, flags, n_limb, cols;
+  const float* x;
+};
+template <class F, int Q>
+__global__ void __launch_bounds__(512) moe_front_kernel(MoeFront a) {
+  if (int(blockIdx.x) < a.n_limb) {
+    limb_rows<F, 2, 4, kLimbPairSilu>(a.gate, 2 * a.n_ff, a.cols, a.rb_sh, a.x, a.h, a.per, a.flags, a.up, a.n_ff,
+                                      nullptr, nullptr, int(blockIdx.x), a.n_limb);
+    return;
+  }
+  __shared__ double part[2][kPlainThreads / kWave];
+  const int sub = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  const int r = 2 * (int(blockIdx.x) - a.n_limb) + sub;
+  const bool tail = r >= a.rows, on = r <= a.rows;
+  const uint8_t* row = tail ? a.w2 : a.w + int64_t(r) * a.rb;
+  double acc = 0.0;
+  constexpr int kStep = kPlainThreads * kPlainUnroll;
+  for (int c0 = 0; c0 < a.cols; c0 += kStep) {
+    float wv[kPlainUnroll], xv[kPlainUnroll];
+#pragma unroll
+    for (int k = 0; k < kPlainUnroll; ++k) {
+      const int c = min(c0 + k * kPlainThreads + tid, a.cols - 1);
+      wv[k] = plain_at<Q>(row, c);
+      const float v = a.x[c];
+      xv[k] = tail ? v : bf16_rne(v);
+    }
+#pragma unroll
+    for (int k = 0; k < kPlainUnroll; ++k)
+      if (c0 + k * kPlainThreads + tid < a.cols) acc = __builtin_fma(double(wv[k]), double(xv[k]), acc);
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, kWave);
+  if (lane == 0) part[sub][wave] = acc;
+  __syncthreads();
+  if (tid == 0 && on) {
+    double v = part[sub][0];
+#pragma unroll
+    for (int k = 1; k < kPlainThreads / kWave; ++k) v += part[sub][k];
+    if (tail) *a.y2 = float(v);
+    else a.y[r] = float(v);
   }
 }
 
@@ -1116,6 +1180,60 @@ hipError_t launch_gemv_plain_pair(uint32_t quant, const void* w1, int64_t rows1,
   }
 }
 
+// Rows of one window (Q6_K: of less, whole windows have a form of their own)
+// and a plain router and gate input of one type.
+bool moe_front_ok(uint32_t q_plain, uint32_t q_gu, int64_t n_expert, int64_t n_embd, int64_t n_ff) {
+  return plain_quant(q_plain) && n_embd <= 4096 && !(q_gu == kQ6_K && n_embd == 4096) && n_embd % 64 == 0 &&
+         (q_gu == kQ4_K || q_gu == kQ8_0 || q_gu == kQ5_K || q_gu == kQ6_K) &&
+         gemv_shape_ok(q_plain, n_expert + 1, n_embd, 1) && gemv_shape_ok(q_gu, 2 * n_ff, n_embd, 1) &&
+         n_ff <= (int64_t(1) << 24) && n_expert <= (int64_t(1) << 24);
+}
+
+template <class F>
+static void launch_front(uint32_t q, const MoeFront& a, unsigned blocks, hipStream_t s) {
+  const size_t lds = size_t(limb_lds_bytes(a.cols));
+  switch (q) {
+    case kF32: hipLaunchKernelGGL((moe_front_kernel<F, kF32>), dim3(blocks), dim3(512), lds, s, a); break;
+    case kF16: hipLaunchKernelGGL((moe_front_kernel<F, kF16>), dim3(blocks), dim3(512), lds, s, a); break;
+    default: hipLaunchKernelGGL((moe_front_kernel<F, kBF16>), dim3(blocks), dim3(512), lds, s, a);
+  }
+}
+
+hipError_t launch_moe_front(uint32_t q_plain, const void* router, int64_t n_expert, const void* gate_inp,
+                            uint32_t q_gu, const void* gate, const void* up, int64_t n_ff, int64_t n_embd,
+                            const float* x, float* logits, float* sg, float* h, int q6, hipStream_t s) {
+  if (!moe_front_ok(q_plain, q_gu, n_expert, n_embd, n_ff)) return hipErrorInvalidValue;
+  const uintptr_t al = uintptr_t(q_plain == kF32 ? 3 : 1);
+  if ((reinterpret_cast<uintptr_t>(router) | reinterpret_cast<uintptr_t>(gate_inp)) & al) return hipErrorInvalidValue;
+  MoeFront a{};
+  a.w = static_cast<const uint8_t*>(router);
+  a.w2 = static_cast<const uint8_t*>(gate_inp);
+  a.rows = int(n_expert);
+  a.rb = byte_size(q_plain, n_embd);
+  a.y = logits;
+  a.y2 = sg;
+  a.gate = static_cast<const uint8_t*>(gate);
+  a.up = static_cast<const uint8_t*>(up);
+  a.n_ff = int(n_ff);
+  a.rb_sh = byte_size(q_gu, n_embd);
+  a.h = h;
+  a.flags = q6;
+  a.cols = int(n_embd);
+  a.x = x;
+  // 8 waves per CU, as launch_shexp_one's gate and up
+  const int n_rg = int(n_ff), waves = 8 * cu_count();
+  a.per = std::min((n_rg + waves - 1) / waves, kLimbMaxRowsOneWin);
+  a.n_limb = ((n_rg + a.per - 1) / a.per + 7) / 8;
+  const unsigned blocks = unsigned(a.n_limb + (a.rows + 2) / 2);
+  switch (q_gu) {
+    case kQ4_K: launch_front<LimbQ4K>(q_plain, a, blocks, s); break;
+    case kQ8_0: launch_front<LimbQ8>(q_plain, a, blocks, s); break;
+    case kQ5_K: launch_front<LimbQ5K>(q_plain, a, blocks, s); break;
+    default: launch_front<LimbQ6K>(q_plain, a, blocks, s);
+  }
+  return hipGetLastError();
+}
+
 // The shared expert of a MoE layer for one token in two limb launches: [g; u]
 // = [gate; up] . x (one launch, x staged once), then d = down . (silu(g) * u)
 // with silu(g) * u formed as the down launch stages its x.
@@ -1128,18 +1246,18 @@ bool shexp_fused_ok(uint32_t q_gu, uint32_t q_d, int64_t n_embd, int64_t n_ff) {
 
 hipError_t launch_shexp_one(uint32_t q_gu, uint32_t q_d, const void* gate, const void* up, const void* down,
                             int64_t n_embd, int64_t n_ff, const float* x, float* gu, float* d, int q6gu, int q6d,
-                            hipStream_t s) {
+                            hipStream_t s, bool h_there) {
   if (!shexp_fused_ok(q_gu, q_d, n_embd, n_ff)) return hipErrorInvalidValue;
   const auto* g = static_cast<const uint8_t*>(gate);
   const auto* u = static_cast<const uint8_t*>(up);
   const auto* w = static_cast<const uint8_t*>(down);
   const int64_t rb1 = byte_size(q_gu, n_embd), rb2 = byte_size(q_d, n_ff);
   const int E = int(n_embd), N = int(n_ff);
-  hipError_t e;
+  hipError_t e = hipSuccess;
   if (E <= 4096) {
     // gate and up in one launch, a gate row and an up row per item, storing
     // h = silu(g) * u (gu[0, N)); down stages h as its x
-    switch (q_gu) {
+    if (!h_there) switch (q_gu) {
       case kQ4_K: e = launch_limb<LimbQ4K, 2, 4, kLimbPairSilu>(g, 2 * N, E, rb1, x, gu, s, 512, 8, q6gu, u, N); break;
       case kQ8_0: e = launch_limb<LimbQ8, 2, 4, kLimbPairSilu>(g, 2 * N, E, rb1, x, gu, s, 512, 8, q6gu, u, N); break;
       case kQ5_K: e = launch_limb<LimbQ5K, 2, 4, kLimbPairSilu>(g, 2 * N, E, rb1, x, gu, s, 512, 8, q6gu, u, N); break;

@@ -55,7 +55,14 @@ hipError_t launch_gemv_plain_pair(uint32_t quant, const void* w1, int64_t rows1,
 bool shexp_fused_ok(uint32_t q_gu, uint32_t q_d, int64_t n_embd, int64_t n_ff);
 hipError_t launch_shexp_one(uint32_t q_gu, uint32_t q_d, const void* gate, const void* up, const void* down,
                             int64_t n_embd, int64_t n_ff, const float* x, float* gu, float* d, int q6gu, int q6d,
-                            hipStream_t s);
+                            hipStream_t s, bool h_there = false);
+// One token: logits = router . bf16(x), sg = gate_inp . x and the shared
+// expert's h = silu(gate . x) * (up . x) in one launch; launch_shexp_one with
+// `h_there` (gu = h) is then its down alone.
+bool moe_front_ok(uint32_t q_plain, uint32_t q_gu, int64_t n_expert, int64_t n_embd, int64_t n_ff);
+hipError_t launch_moe_front(uint32_t q_plain, const void* router, int64_t n_expert, const void* gate_inp,
+                            uint32_t q_gu, const void* gate, const void* up, int64_t n_ff, int64_t n_embd,
+                            const float* x, float* logits, float* sg, float* h, int q6, hipStream_t s);
 
 // Batch 2..8 of Q4_K or Q5_K rows on int8 MFMA (exact integer
 // activations, staged in LDS 4096 columns at a time); `cu` is the device's

@@ -143,3 +143,37 @@ def test_moe_layer_many_tokens(n_sh, n_tok):
         assert np.array_equal(out.cpu().numpy(), got), rep
         call(0, 4, few)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("plain,n_expert,n_embd,n_sh,q_sh", [
+    (0, 5, 768, 256, Q4_K), (0, 16, 4096, 768, Q5_K), (1, 7, 512, 4608, Q8_0), (30, 12, 2304, 256, Q6_K)])
+def test_moe_layer_one_token_front(plain, n_expert, n_embd, n_sh, q_sh):
+    """One token: router, gate input and the shared expert's gate and up in
+    one launch (odd and even row counts, every plain type and a row pair per
+    wave or several), against the two-token call's first token, which takes
+    them apart."""
+    import torch
+    print("[case] moe layer front", plain, n_expert, n_embd, n_sh, q_sh, flush=True)
+    n_ff, top_k = 256, 4
+    q, t = layer_om_tensors(n_expert, n_embd, n_ff, n_sh, 190 + n_expert)
+    q, t = list(q), list(t)
+    for i in (0, 7):
+        q[i] = plain
+        f = torch.from_numpy(t[i].view(np.float32).copy())
+        t[i] = (f if plain == 0 else f.to(torch.float16 if plain == 1 else torch.bfloat16)).view(torch.uint8).numpy()
+    for i, (r, c) in ((4, (n_sh, n_embd)), (5, (n_sh, n_embd))):
+        q[i], t[i] = q_sh, S.matrix(q_sh, 200 + i, r, c)
+    x = S.normal_f32(191, 2 * n_embd).reshape(2, n_embd)
+    bufs = [torch.from_numpy(np.ascontiguousarray(a).reshape(-1)).cuda() for a in t]
+    flags = [0, OM, OM, OM, 0, 0, 0, 0]
+    tx = torch.from_numpy(x).cuda()
+    res = []
+    for n in (1, 2):
+        out = torch.full((n, n_embd), float("nan"), device="cuda")
+        nb = H.moe_layer_workspace_bytes(n, top_k, n_expert, n_embd, n_ff, n_sh, q)
+        ws = torch.full((nb,), 0xFF, dtype=torch.uint8, device="cuda")
+        H.moe_layer_dev([(q[i], flags[i], bufs[i].data_ptr()) for i in range(8)], n_expert, n_embd, n_ff, n_sh, n, top_k,
+                        tx.data_ptr(), out.data_ptr(), ws.data_ptr(), nb, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        res.append(out.cpu().numpy()[0])
+    check_parity(res[0], res[1], "token 0", strict_tol=2 * STRICT_TOL)
