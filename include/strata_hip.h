@@ -428,7 +428,8 @@ int sh_upload_gguf_tensor(sh_context* ctx, const sh_gguf* gguf, uint64_t index, 
  * h = g / (1 + exp(-g)) * u (f32); out = x + down . h (f32). tensors[3]:
  * gate, up [n_ff][n_embd] and down [n_embd][n_ff], any matvec types; x, out
  * [n_tok][n_embd] (out may equal x: the residual add in place); post_norm
- * [n_embd]; workspace >= sh_ffn_workspace_bytes, 256-byte aligned. One token
+ * [n_embd]; workspace of sh_ffn_workspace_bytes, 256-byte aligned (one for
+ * more tokens serves fewer, if not always at the full speed). One token
  * with one quantized type runs in three launches (rms_norm; gate and up
  * together; down with silu(g) * u staged and the residual added). No
  * reference counterpart as one call: it replaces the six steps above. */

@@ -1495,11 +1495,11 @@ static int ffn_dev_check(const sh_expert_dev* t, uint64_t n_embd, uint64_t n_ff,
 
 static hipError_t ffn_dev_launch(const sh_expert_dev* t, uint64_t n_embd, uint64_t n_ff, uint32_t n_tok,
                                  const float* x, const float* post_norm, double eps, float* out, void* workspace,
-                                 void* stream) {
+                                 size_t workspace_bytes, void* stream) {
   auto q6 = [](const sh_expert_dev& d) { return reading(d.quant, d.flags); };
   return sh::launch_ffn(t[0].quant, t[1].quant, t[2].quant, t[0].data, t[1].data, t[2].data, q6(t[0]),
                         q6(t[1]), q6(t[2]), int64_t(n_embd), int64_t(n_ff), int(n_tok), x, post_norm, eps,
-                        out, workspace, static_cast<hipStream_t>(stream));
+                        out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 int sh_ffn_dev(const sh_expert_dev* t, uint64_t n_embd, uint64_t n_ff, uint32_t n_tok, const float* x,
@@ -1509,12 +1509,14 @@ int sh_ffn_dev(const sh_expert_dev* t, uint64_t n_embd, uint64_t n_ff, uint32_t 
   int rc = ffn_dev_check(t, n_embd, n_ff, n_tok, x, post_norm, out, &need);
   if (rc) return rc;
   if (!workspace) return fail(SH_ERR_INVALID_ARGUMENT, "null workspace");
+  need = sh::ffn_workspace_min(n_tok, int64_t(n_embd), int64_t(n_ff));
   if (workspace_bytes < need)
     return fail(SH_ERR_INVALID_ARGUMENT, "workspace of %llu bytes, %llu needed", (unsigned long long)workspace_bytes,
                 (unsigned long long)need);
   if (reinterpret_cast<uintptr_t>(workspace) & 255u)
     return fail(SH_ERR_INVALID_ARGUMENT, "workspace must be 256-byte aligned");
-  HIP_TRY(ffn_dev_launch(t, n_embd, n_ff, n_tok, x, post_norm, eps, out, workspace, stream), "ffn launch");
+  HIP_TRY(ffn_dev_launch(t, n_embd, n_ff, n_tok, x, post_norm, eps, out, workspace, size_t(workspace_bytes), stream),
+          "ffn launch");
   return SH_OK;
 }
 
@@ -1548,7 +1550,7 @@ int sh_ffn_dev_noalloc(const sh_expert_dev* t, uint64_t n_embd, uint64_t n_ff, u
                 (unsigned long long)kScratchBytes);
   void* ws = nullptr;
   if ((rc = scratch_address(&ws))) return rc;
-  HIP_TRY(ffn_dev_launch(t, n_embd, n_ff, n_tok, x, post_norm, eps, out, ws, stream), "ffn launch");
+  HIP_TRY(ffn_dev_launch(t, n_embd, n_ff, n_tok, x, post_norm, eps, out, ws, kScratchBytes, stream), "ffn launch");
   return SH_OK;
 }
 
@@ -1595,7 +1597,7 @@ int sh_ffn(sh_context* c, const sh_quant_tensor* gate, const sh_quant_tensor* up
   HIP_TRY(sh::launch_ffn(gate->quant, up->quant, down->quant, dev[0], dev[1], dev[2],
                          reading(gate->quant, gate->flags), reading(up->quant, up->flags),
                          reading(down->quant, down->flags), int64_t(n_embd), int64_t(n_ff), int(n_tok), dx, dn, eps, dx, c->d_blk.p,
-                         c->stream),
+                         size_t(need), c->stream),
           "ffn launch");
   HIP_TRY(sh::launch_copy_bytes(dx, c->h_out.dev, xb, c->stream), "x readback");
   HIP_TRY(hipStreamSynchronize(c->stream), "ffn");

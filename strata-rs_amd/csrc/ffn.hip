@@ -55,6 +55,8 @@ constexpr int kFfnMaxSplit = 8;
 // takes as many shares as fit, of each product by itself (17 tokens at 4096 /
 // 12288: one share of gate and up fills what is left, but eight of down do not;
 // with one of each the call took 190 us, so 78). Larger ones have room for all it asks for.
+size_t ffn_workspace_min(int64_t n_tok, int64_t n_embd, int64_t n_ff) { return ffn_step_bytes(n_tok, n_embd, n_ff); }
+
 size_t ffn_workspace_bytes(int64_t n_tok, int64_t n_embd, int64_t n_ff) {
   const size_t steps = ffn_step_bytes(n_tok, n_embd, n_ff);
   if (n_tok <= 8 || n_tok > kFfnMaxTokTokens) return steps;
@@ -76,7 +78,8 @@ static hipError_t gemv_rows(uint32_t quant, const void* w, int64_t rows, int64_t
 hipError_t launch_ffn(uint32_t q_gate, uint32_t q_up, uint32_t q_down, const void* gate, const void* up,
                       const void* down, int q6g, int q6u, int q6d, int64_t n_embd, int64_t n_ff, int n_tok,
                       const float* x, const float* post_norm, double eps, float* out, void* workspace,
-                      hipStream_t s) {
+                      size_t workspace_bytes, hipStream_t s) {
+  if (workspace_bytes < ffn_workspace_min(n_tok, n_embd, n_ff)) return hipErrorInvalidValue;
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   const size_t T = size_t(n_tok);
   float* mixed = reinterpret_cast<float*>(ws);
@@ -91,7 +94,9 @@ hipError_t launch_ffn(uint32_t q_gate, uint32_t q_up, uint32_t q_down, const voi
   }
   if (n_tok > 8 && n_tok <= kFfnMaxTokTokens && q_gate == q_up && q6g == q6u && tok_ok(q_gate, n_ff, n_embd) &&
       tok_ok(q_down, n_embd, n_ff)) {
-    const size_t room = ffn_workspace_bytes(n_tok, n_embd, n_ff);
+    // no more than the reported size is used, so results do not depend on
+    // how much more than that a caller has
+    const size_t room = std::min(workspace_bytes, ffn_workspace_bytes(n_tok, n_embd, n_ff));
     int gu_split = kFfnMaxSplit, dn_split = kFfnMaxSplit;
     FfnTok p = ffn_tok_plan(n_tok, n_embd, n_ff, gu_split, 1);
     while (p.bytes > room && gu_split > 1) p = ffn_tok_plan(n_tok, n_embd, n_ff, --gu_split, 1);

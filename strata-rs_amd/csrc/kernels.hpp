@@ -33,14 +33,16 @@ hipError_t launch_ffn_one(uint32_t quant, const void* gate, const void* up, cons
 hipError_t launch_silu_mul(const float* g, const float* u, float* h, int64_t n, hipStream_t stream);
 
 // The dense FFN half of a layer for n_tok tokens (rms_norm, gate, up, silu,
-// down, residual); workspace of ffn_workspace_bytes.
+// down, residual); workspace of ffn_workspace_min at least (with
+// ffn_workspace_bytes many tokens take their fastest form).
 constexpr size_t kFfnFixedScratch = size_t(4) << 20;  // of sh_ffn_dev_noalloc
 constexpr int64_t kFfnMaxTokTokens = 65535;  // tokens of the many-token form (a grid dimension of its conversion)
+size_t ffn_workspace_min(int64_t n_tok, int64_t n_embd, int64_t n_ff);
 size_t ffn_workspace_bytes(int64_t n_tok, int64_t n_embd, int64_t n_ff);
 hipError_t launch_ffn(uint32_t q_gate, uint32_t q_up, uint32_t q_down, const void* gate, const void* up,
                       const void* down, int q6g, int q6u, int q6d, int64_t n_embd, int64_t n_ff, int n_tok,
                       const float* x, const float* post_norm, double eps, float* out, void* workspace,
-                      hipStream_t stream);
+                      size_t workspace_bytes, hipStream_t stream);
 constexpr int kPlainMaxBatch = 1024;
 // The same for F32 / F16 / BF16 rows against bf16(x) (rounded as loaded), for
 // up to kPlainMaxBatch vectors.

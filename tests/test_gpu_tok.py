@@ -85,3 +85,26 @@ def test_ffn_many_tokens_other_reading(oracle, quant, flag):
     got = ffn((quant,) * 3, (flag,) * 3, mats, n_embd, n_ff, x, norm)
     want = oracle.dense_ffn((0, 0, 0), [w.view(np.uint8) for w in f32], n_embd, n_ff, x, norm, 1e-6)
     check_parity(got.astype(np.float64) - x, want.astype(np.float64) - x, "ffn out - x")
+
+
+def test_ffn_workspace_of_more_tokens(oracle):
+    """A workspace reported for n tokens is taken for fewer, and one of the
+    step-by-step form's size (mixed, g and u, h, m) always is."""
+    import torch
+    print("[case] ffn workspace", flush=True)
+    n_embd, n_ff, quants = 512, 768, (Q4_K, Q4_K, Q6_K)
+    mats = [S.matrix(quants[0], 31, n_ff, n_embd), S.matrix(quants[1], 32, n_ff, n_embd),
+            S.matrix(quants[2], 33, n_embd, n_ff)]
+    dev = [torch.from_numpy(m).cuda() for m in mats]
+    norm = S.normal_f32(34, n_embd)
+    nd = torch.from_numpy(norm).cuda()
+    for n_tok, size in ((200, H.ffn_workspace_bytes(201, n_embd, n_ff)), (200, 4 * 200 * (2 * n_embd + 3 * n_ff))):
+        x = S.normal_f32(35, n_tok * n_embd).reshape(n_tok, n_embd)
+        xd = torch.from_numpy(x).cuda()
+        out = torch.full_like(xd, float("nan"))
+        ws = torch.full((size,), 0xFF, dtype=torch.uint8, device="cuda")
+        H.ffn_dev([(q, 0, t.data_ptr()) for q, t in zip(quants, dev)], n_embd, n_ff, n_tok, xd.data_ptr(),
+                  nd.data_ptr(), 1e-6, out.data_ptr(), ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        want = oracle.dense_ffn(quants, mats, n_embd, n_ff, x, norm, 1e-6)
+        check_parity(out.cpu().numpy().astype(np.float64) - x, want.astype(np.float64) - x, "ffn out - x")
