@@ -35,7 +35,7 @@ static TokPlan moe_tok_plan(const MoePlan& p, int rows, int mats, int cols) {
 // moe_om.hip's launches, three fewer and one pass over the weights per two
 // pairs, stay the faster form for few pairs of small experts. Both measured,
 // Q4_K / Q6_K 128 x 2048 x 768 top-8: 4 tokens 59 against 60 us, 8 99 / 75, 16
-// 176 / 97, 96 640 / 169, 256 1465 / 203; Q5_K / Q8_0 32 x 1280 x 512 top-2:
+// 176 / 97, 96 640 / 183, 256 1465 / 214; Q5_K / Q8_0 32 x 1280 x 512 top-2:
 // 8 tokens 29 / 35, 16 39 / 36, 64 81 / 42, 256 242 / 53.
 int moe_tok_group(const MoePlan& p, uint32_t qa, uint32_t qb) {
   if (!tok_ok(qa, p.n_ff, p.n_embd) || !tok_ok(qb, p.n_embd, p.n_ff)) return 0;

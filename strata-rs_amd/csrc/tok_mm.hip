@@ -192,7 +192,8 @@ constexpr bool tok_lds_format() {
 // straight to the lanes (32 rows x 32 bytes each) cost an access or two per
 // lane: Q6_K down of 96 tokens x 8 of 128 experts took 36 M accesses for 165
 // MB, and the load unit bound it. Routed FFN, 128 x 2048 x 768 Q4_K / Q6_K: 16
-// tokens 111 -> 98 us, 64 189 -> 155, 96 204 -> 169, 256 231 -> 214; dense FFN
+// tokens 111 -> 98 us, 64 189 -> 155 to 170, 96 204 -> 169 to 186, 256 231 ->
+// 214; dense FFN
 // 2048 / 6144 Q5_K / Q8_0, 12 tokens 43 -> 34.
 template <class F, bool CO>
 struct TokWave {
