@@ -1023,16 +1023,37 @@ static hipError_t launch_nb(int nb, const uint8_t* w, int rows, int cols, int64_
 }
 
 // Vectors per launch of gemv_q6win_kernel (as even as they go), 0: a shape it
-// does not take.
+// does not take. It pays where it takes fewer rounds of waves: two rows a wave
+// against one, each of its rounds about 1.4 of gemv_kernel's (4096 x 6144, four
+// vectors, us before and now: 2048 rows, one round of either, 9.7 / 13.9; 4096,
+// two against one, 17.5 / 15.0; 6000, three against two, 22.4 / 22.8; 8192,
+// four against two, 27.1 / 22.7). It takes four vectors at most, so it needs no
+// more launches than gemv_kernel does, which takes eight where LDS holds them,
+// or so many rows that a launch more costs less than it saves (x 4096, us: 8192
+// rows, 8 vectors 29.2 / 27.9, 7 26.1 / 25.9, 6 23.6 / 24.4; 10240, half a
+// round left over, 8 34.4 / 36.3; 32768, 8 89.8 / 80.1, 7 79.7 / 76.2, 6 70.3
+// / 72.1; 65536, 6 131 / 121, 5 114 / 112). A vector by itself that
+// gemv_kernel leaves over takes the batch-1 form, which costs less than a pair
+// (8192 x 8192, 5 vectors as 4 + 1 40.0, as 3 + 2 40.9).
 static size_t q6win_lds(int cols, int nb, int waves) {
   return size_t(nb) * xw_stride(cols) * sizeof(float) + size_t(waves) * 2 * kWinQ6;
 }
-static int q6win_batch(const uint8_t* w, int cols, int batch) {
+static int q6win_batch(const uint8_t* w, int rows, int cols, int batch) {
   if (batch < 2 || cols % 2048 != 0 || (reinterpret_cast<uintptr_t>(w) & 15u)) return 0;
+  // rounds of gemv_kernel's waves (a sixteenth of a round does not count) and of this form's
+  const int64_t round = 8 * cu_count();
+  const int64_t one = (rows + round - round / 16 - 1) / round, two = (rows + 2 * round - 1) / (2 * round);
+  if (3 * two >= 2 * one) return 0;
   int most = 4;
   while (most >= 2 && q6win_lds(cols, most, 8) > kMaxLds) --most;
   if (most < 2) return 0;
   const int n = (batch + most - 1) / most, per = (batch + n - 1) / n;
+  const int held = std::min(8, int(kMaxLds / lds_bytes(cols, 1))), before = (batch + held - 1) / held;
+  if (n > before) {
+    const int64_t many = batch == 8 ? 4 : batch == 7 ? 16 : batch == 6 ? 32 : 1 << 30;
+    if (before > 1 || n > 2 || rows < many * round || 9 * two > 5 * one) return 0;
+  }
+  if (batch % held == 1 && 3 * n > batch) return 0;
   // (the last launch takes what is left, at least two)
   return batch - (n - 1) * per >= 2 || n == 1 ? per : 0;
 }
@@ -1082,7 +1103,7 @@ hipError_t launch_gemv(uint32_t quant, const void* wv, int64_t rows, int64_t col
     return hipErrorInvalidValue;
   if (batch >= 2 && gemv_mfma_ok(quant, rows, cols, batch))
     return launch_gemv_mfma(quant, w, rows, cols, x, y, batch, cu_count(), stream, ws);
-  if (const int per = quant == kQ6_K ? q6win_batch(w, int(cols), batch) : 0) {
+  if (const int per = quant == kQ6_K ? q6win_batch(w, int(rows), int(cols), batch) : 0) {
     for (int b0 = 0; b0 < batch; b0 += per) {
       const float* xb = x + int64_t(b0) * cols;
       float* yb = y + int64_t(b0) * rows;
