@@ -221,7 +221,9 @@ __global__ void __launch_bounds__(64 * kWinWaves)
     for (int b = 0; b < NB; ++b) acc[i][b] = 0.f;
   while (rg < n_rg) {
     // into LDS (a wave's LDS operations run in order: its reads below see
-    // every lane's pieces, its next writes come after them)
+    // every lane's pieces, its next writes come after them; the fences hold
+    // the compiler to that order, as other lanes' reads are no reason to it)
+    asm volatile("" ::: "memory");
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -229,6 +231,8 @@ __global__ void __launch_bounds__(64 * kWinWaves)
         const int off = 16 * lane + 1024 * k;
         if (off < kWinQ6) *reinterpret_cast<u32x4*>(buf + i * kWinQ6 + off) = p[i][k];
       }
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
     int nrg = rg, nwn = win + 1;
     if (nwn == nwin) {
       nwn = 0;
