@@ -279,7 +279,8 @@ int sh_matmul(sh_context* ctx, const sh_quant_tensor* w, const float* x, uint32_
 
 /* Bytes of device workspace sh_matmul_dev uses: the converted activations,
  * and, where the output's tiles are too few for the chip, the partial sums
- * of columns split over more workgroups. */
+ * of columns split over more workgroups. As every size query: arithmetic, the
+ * same on every device, without a call into the HIP runtime. */
 int sh_matmul_workspace_bytes(uint32_t quant, uint64_t rows, uint64_t cols, uint32_t m, uint32_t mode,
                               uint64_t* bytes);
 

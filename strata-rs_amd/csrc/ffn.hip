@@ -39,10 +39,10 @@ struct FfnTok {
   TokPlan gu, dn;
   size_t o_part, bytes;
 };
-static FfnTok ffn_tok_plan(int64_t n_tok, int64_t n_embd, int64_t n_ff, int gu_split, int dn_split) {
+static FfnTok ffn_tok_plan(int64_t n_tok, int64_t n_embd, int64_t n_ff, int cu, int gu_split, int dn_split) {
   FfnTok p{};
-  p.gu = tok_plan(n_ff, 2, n_embd, int(n_tok), cu_count(), gu_split);
-  p.dn = tok_plan(n_embd, 1, n_ff, int(n_tok), cu_count(), dn_split);
+  p.gu = tok_plan(n_ff, 2, n_embd, int(n_tok), cu, gu_split);
+  p.dn = tok_plan(n_embd, 1, n_ff, int(n_tok), cu, dn_split);
   const size_t T = size_t(n_tok) * sizeof(float);
   p.o_part = align256(std::max(tok_image_bytes(p.gu), tok_image_bytes(p.dn)));
   p.bytes = p.o_part + align256(std::max({T * n_embd, T * 2 * n_ff * p.gu.nsplit, T * n_embd * p.dn.nsplit}));
@@ -60,7 +60,7 @@ size_t ffn_workspace_min(int64_t n_tok, int64_t n_embd, int64_t n_ff) { return f
 size_t ffn_workspace_bytes(int64_t n_tok, int64_t n_embd, int64_t n_ff) {
   const size_t steps = ffn_step_bytes(n_tok, n_embd, n_ff);
   if (n_tok <= 8 || n_tok > kFfnMaxTokTokens) return steps;
-  const size_t tok = ffn_tok_plan(n_tok, n_embd, n_ff, kFfnMaxSplit, kFfnMaxSplit).bytes;
+  const size_t tok = ffn_tok_plan(n_tok, n_embd, n_ff, kChipCus, kFfnMaxSplit, kFfnMaxSplit).bytes;
   return std::max(steps, steps <= kFfnFixedScratch ? std::min(tok, kFfnFixedScratch) : tok);
 }
 
@@ -98,10 +98,11 @@ hipError_t launch_ffn(uint32_t q_gate, uint32_t q_up, uint32_t q_down, const voi
     // how much more than that a caller has
     const size_t room = std::min(workspace_bytes, ffn_workspace_bytes(n_tok, n_embd, n_ff));
     int gu_split = kFfnMaxSplit, dn_split = kFfnMaxSplit;
-    FfnTok p = ffn_tok_plan(n_tok, n_embd, n_ff, gu_split, 1);
-    while (p.bytes > room && gu_split > 1) p = ffn_tok_plan(n_tok, n_embd, n_ff, --gu_split, 1);
-    p = ffn_tok_plan(n_tok, n_embd, n_ff, gu_split, dn_split);
-    while (p.bytes > room && dn_split > 1) p = ffn_tok_plan(n_tok, n_embd, n_ff, gu_split, --dn_split);
+    const int cu = cu_count();
+    FfnTok p = ffn_tok_plan(n_tok, n_embd, n_ff, cu, gu_split, 1);
+    while (p.bytes > room && gu_split > 1) p = ffn_tok_plan(n_tok, n_embd, n_ff, cu, --gu_split, 1);
+    p = ffn_tok_plan(n_tok, n_embd, n_ff, cu, gu_split, dn_split);
+    while (p.bytes > room && dn_split > 1) p = ffn_tok_plan(n_tok, n_embd, n_ff, cu, gu_split, --dn_split);
     if (p.bytes <= room) {
       float* part = reinterpret_cast<float*>(ws + p.o_part);
       const int64_t nx = int64_t(T) * n_embd, ng = int64_t(T) * 2 * n_ff;

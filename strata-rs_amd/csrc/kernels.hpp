@@ -255,6 +255,10 @@ hipError_t launch_tok_mm(const TokPlan& p, uint32_t quant, const void* w0, const
 hipError_t launch_tok_sum(const float* part, int64_t stride, int nsplit, const float* res, float* out, int64_t n,
                           hipStream_t s);
 int cu_count();  // of the current device
+// The CUs of a whole chip, for the workspace sizes: those are arithmetic, the
+// same on every device and without a call into the HIP runtime; a launch takes
+// the device's own count and as many shares as the workspace it was given holds.
+constexpr int kChipCus = 256;
 
 // The trait's elementwise methods over `rows` rows of n floats (rope:
 // head_dim floats per row, row r at position pos0 + r / heads_per_pos).

@@ -1654,11 +1654,11 @@ static size_t mm_act_bytes(int64_t cols, int64_t m, uint32_t mode) {
 struct MmShape {
   int bm, shares, c_per;  // c_per: chunks of a share, whole super-blocks
 };
-static MmShape mm_shape(uint32_t quant, int64_t rows, int64_t cols, int64_t m, uint32_t mode, size_t room) {
+static MmShape mm_shape(uint32_t quant, int64_t rows, int64_t cols, int64_t m, uint32_t mode, int64_t cu, size_t room) {
   const int nch = int(cols / kMmKC);
   MmShape best{kMmBM, 1, (nch + 3) / 4 * 4};
   if (mode == 2) return best;
-  const int64_t cu = cu_count(), rt = (rows + kMmBN - 1) / kMmBN;
+  const int64_t rt = (rows + kMmBN - 1) / kMmBN;
   const double part_us = double(m) * double(rows) * 8.0 / 4e6;  // a share's sums written and read
   double best_t = 0;
   for (int bm = kMmBM; bm >= kMmBM / 2; bm /= 2) {
@@ -1684,7 +1684,7 @@ size_t matmul_workspace_min(int64_t cols, int64_t m, uint32_t mode) { return mm_
 
 size_t matmul_workspace_bytes(uint32_t quant, int64_t rows, int64_t cols, int64_t m, uint32_t mode) {
   const size_t act = mm_act_bytes(cols, m, mode);
-  const MmShape sh = mm_shape(quant, rows, cols, m, mode, ~size_t(0));
+  const MmShape sh = mm_shape(quant, rows, cols, m, mode, kChipCus, ~size_t(0));
   return act + (sh.shares > 1 ? mm_part_bytes(rows, m, sh.shares) : 0);
 }
 
@@ -1757,7 +1757,7 @@ hipError_t launch_matmul(uint32_t quant, const void* wv, int64_t rows, int64_t c
   if (!matmul_shape_ok(quant, rows, cols, m, mode)) return hipErrorInvalidValue;
   const size_t act = mm_act_bytes(cols, m, mode);
   if (workspace_bytes < act) return hipErrorInvalidValue;
-  const MmShape sh = mm_shape(quant, rows, cols, m, mode, workspace_bytes - act);
+  const MmShape sh = mm_shape(quant, rows, cols, m, mode, cu_count(), workspace_bytes - act);
   const uint8_t* w = static_cast<const uint8_t*>(wv);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   const int64_t rb = byte_size(quant, cols);

@@ -83,8 +83,8 @@ bool moe_layer_plan(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, in
   p.sh_tok = n_tok > 8 && q.gate_sh == q.up_sh && tok_ok(q.gate_sh, n_ff_sh, n_embd) &&
              tok_ok(q.down_sh, n_embd, n_ff_sh);
   if (p.sh_tok) {
-    const TokPlan gu = tok_plan(n_ff_sh, 2, n_embd, n_tok, cu_count(), kShMaxSplit);
-    const TokPlan dn = tok_plan(n_embd, 1, n_ff_sh, n_tok, cu_count(), kShMaxSplit);
+    const TokPlan gu = tok_plan(n_ff_sh, 2, n_embd, n_tok, kChipCus, kShMaxSplit);
+    const TokPlan dn = tok_plan(n_embd, 1, n_ff_sh, n_tok, kChipCus, kShMaxSplit);
     p.o_sh_img = take(std::max(tok_image_bytes(gu), tok_image_bytes(dn)));
     // as for kShMaxSplit shares, whatever the plans take: more tokens never
     // need less
