@@ -321,8 +321,9 @@ int sh_moe_workspace_bytes(uint32_t n_tok, uint32_t top_k, uint64_t n_expert, ui
                            uint64_t* bytes);
 
 /* sh_moe_ffn on device pointers; logits, x, out and workspace are device
- * buffers, workspace at least sh_moe_workspace_bytes() long and 256-byte
- * aligned. Calls sharing one workspace must not overlap in time. */
+ * buffers, workspace of sh_moe_workspace_bytes(), 256-byte aligned (one that
+ * holds the two-token form alone is taken too, at that form's speed; it sums
+ * in another order). Calls sharing one workspace must not overlap in time. */
 int sh_moe_ffn_dev(const sh_expert_dev* gate, const sh_expert_dev* up, const sh_expert_dev* down,
                    uint64_t n_expert, uint64_t n_embd, uint64_t n_ff, const float* logits,
                    uint32_t n_tok, uint32_t top_k, const float* x, float* out, void* workspace,
@@ -337,9 +338,9 @@ int sh_moe_layer_workspace_bytes(uint32_t n_tok, uint32_t top_k, uint64_t n_expe
 /* sh_moe_layer on device pointers: tensors[8] in the order router, gate,
  * up, down (expert tensors, as in sh_moe_ffn_dev), gate_shexp, up_shexp,
  * down_shexp, gate_inp_shexp (row-major matrices); x (16-byte aligned) and
- * out [n_tok][n_embd]; workspace at least sh_moe_layer_workspace_bytes()
- * long and 256-byte aligned. Calls sharing one workspace must not overlap
- * in time. */
+ * out [n_tok][n_embd]; workspace of sh_moe_layer_workspace_bytes(), 256-byte
+ * aligned (one without room for the many-token forms is taken too, as in
+ * sh_moe_ffn_dev). Calls sharing one workspace must not overlap in time. */
 int sh_moe_layer_dev(const sh_expert_dev* tensors, uint64_t n_expert, uint64_t n_embd, uint64_t n_ff,
                      uint64_t n_ff_shexp, uint32_t n_tok, uint32_t top_k, const float* x, float* out,
                      void* workspace, uint64_t workspace_bytes, void* stream);

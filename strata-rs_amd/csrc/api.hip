@@ -572,7 +572,8 @@ static int mixed_orientation() {
 }
 
 static int moe_check(uint64_t n_expert, uint64_t n_embd, uint64_t n_ff, uint32_t n_tok,
-                     uint32_t top_k, uint32_t qa, uint32_t qb, sh::MoePlan* plan, bool out_major = false) {
+                     uint32_t top_k, uint32_t qa, uint32_t qb, sh::MoePlan* plan, bool out_major = false,
+                     bool tokens = true) {
   if (n_expert == 0 || n_expert > uint64_t(sh::kMoeMaxExperts))
     return fail(SH_ERR_UNSUPPORTED_SHAPE, "n_expert %llu outside 1..%d", (unsigned long long)n_expert,
                 sh::kMoeMaxExperts);
@@ -582,7 +583,8 @@ static int moe_check(uint64_t n_expert, uint64_t n_embd, uint64_t n_ff, uint32_t
     return fail(SH_ERR_UNSUPPORTED_SHAPE, "n_tok %u outside 1..%d", n_tok, sh::kMoeMaxTokens);
   if (n_embd > (1u << 20) || n_ff > (1u << 20))
     return fail(SH_ERR_UNSUPPORTED_SHAPE, "MoE widths too large");
-  if (!sh::moe_plan(int(n_tok), int(top_k), int(n_expert), int(n_embd), int(n_ff), qa, qb, plan, out_major))
+  if (!sh::moe_plan(int(n_tok), int(top_k), int(n_expert), int(n_embd), int(n_ff), qa, qb, plan, out_major,
+                    tokens))
     return fail(SH_ERR_UNSUPPORTED_SHAPE, "MoE %llu x %llu (types %u, %u, %s) is not supported",
                 (unsigned long long)n_embd, (unsigned long long)n_ff, qa, qb, out_major ? "out-major" : "in-major");
   return SH_OK;
@@ -678,14 +680,15 @@ int sh_moe_ffn(sh_context* c, const sh_expert_view* gate, const sh_expert_view* 
 // gate_inp_shexp [1][n_embd]; then the plan.
 static int moe_layer_check(uint64_t E, uint64_t n_embd, uint64_t n_ff, uint64_t n_sh, uint32_t n_tok,
                            uint32_t top_k, const sh::MoeLayerTypes& q, sh::MoeLayerPlan* plan,
-                           bool out_major = false) {
-  int rc = moe_check(E, n_embd, n_ff, n_tok, top_k, q.gate, q.down, &plan->moe, out_major);
+                           bool out_major = false, bool tokens = true, bool sh_tokens = true) {
+  int rc = moe_check(E, n_embd, n_ff, n_tok, top_k, q.gate, q.down, &plan->moe, out_major, tokens);
   if (rc) return rc;
   if (q.up != q.gate)
     return fail(SH_ERR_UNSUPPORTED_QUANT, "gate (%u) and up (%u) types differ", q.gate, q.up);
   if (n_sh == 0 || n_sh > (1u << 20)) return fail(SH_ERR_UNSUPPORTED_SHAPE, "shared expert width %llu",
                                                  (unsigned long long)n_sh);
-  if (!sh::moe_layer_plan(int(n_tok), int(top_k), int(E), int(n_embd), int(n_ff), int(n_sh), q, plan, out_major))
+  if (!sh::moe_layer_plan(int(n_tok), int(top_k), int(E), int(n_embd), int(n_ff), int(n_sh), q, plan, out_major,
+                          tokens, sh_tokens))
     return fail(SH_ERR_UNSUPPORTED_SHAPE,
                 "MoE layer: router %llux%llu (type %u) or shared expert %llu wide (types %u, %u, %u, gate %u) "
                 "is not a matvec shape the kernels take",
@@ -956,6 +959,10 @@ int sh_moe_ffn_dev(const sh_expert_dev* gate, const sh_expert_dev* up, const sh_
   sh::MoePlan plan;
   int rc = moe_check(n_expert, n_embd, n_ff, n_tok, top_k, gate->quant, down->quant, &plan, om == 1);
   if (rc) return rc;
+  // the many-token form where its workspace is there
+  if (workspace_bytes < plan.bytes &&
+      (rc = moe_check(n_expert, n_embd, n_ff, n_tok, top_k, gate->quant, down->quant, &plan, om == 1, false)))
+    return rc;
   if (workspace_bytes < plan.bytes)
     return fail(SH_ERR_INVALID_ARGUMENT, "workspace of %llu bytes, %llu needed",
                 (unsigned long long)workspace_bytes, (unsigned long long)plan.bytes);
@@ -1016,6 +1023,10 @@ int sh_moe_layer_dev(const sh_expert_dev* t, uint64_t n_expert, uint64_t n_embd,
     if ((rc = check_matrix(t[i].quant, dims[i][0], dims[i][1], 1, ~uint64_t(0), i == 0 || i >= 4))) return rc;
   sh::MoeLayerPlan plan;
   if ((rc = moe_layer_check(n_expert, n_embd, n_ff, n_ff_shexp, n_tok, top_k, q, &plan, om == 1))) return rc;
+  // the many-token forms where their workspace is there
+  for (int routed = 1; routed >= 0 && workspace_bytes < plan.bytes; --routed)
+    if ((rc = moe_layer_check(n_expert, n_embd, n_ff, n_ff_shexp, n_tok, top_k, q, &plan, om == 1, routed, false)))
+      return rc;
   if (workspace_bytes < plan.bytes)
     return fail(SH_ERR_INVALID_ARGUMENT, "workspace of %llu bytes, %llu needed",
                 (unsigned long long)workspace_bytes, (unsigned long long)plan.bytes);

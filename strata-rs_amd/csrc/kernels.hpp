@@ -131,11 +131,12 @@ struct MoePlan {
 };
 
 // out_major: gate / up [n_expert][n_ff][n_embd] and down [n_expert][n_embd]
-// [n_ff] (llama.cpp's stacks) instead of [n_expert][in][out].
+// [n_ff] (llama.cpp's stacks) instead of [n_expert][in][out]. `tokens` false:
+// without the many-token form (moe_tok.hip), which needs the larger workspace.
 bool moe_plan(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, uint32_t q_gateup,
-              uint32_t q_down, MoePlan* plan, bool out_major = false);
+              uint32_t q_down, MoePlan* plan, bool out_major = false, bool tokens = true);
 bool moe_plan_out_major(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, uint32_t q_gateup,
-                        uint32_t q_down, MoePlan* plan);
+                        uint32_t q_down, MoePlan* plan, bool tokens);
 // The gate/up and down launches of an out-major plan (route and combine as
 // launch_moe's).
 void launch_moe_out_major(const MoePlan& p, uint32_t qg, uint32_t qd, const void* gate, const void* up,
@@ -195,8 +196,11 @@ struct MoeLayerPlan {
   size_t o_sh_img, o_sh_part;
   size_t bytes;
 };
+// `tokens`, `sh_tokens` false: without the many-token form of the routed
+// experts, of the shared one.
 bool moe_layer_plan(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, int n_ff_sh,
-                    const MoeLayerTypes& q, MoeLayerPlan* plan, bool out_major = false);
+                    const MoeLayerTypes& q, MoeLayerPlan* plan, bool out_major = false, bool tokens = true,
+                    bool sh_tokens = true);
 hipError_t launch_moe_layer(const MoeLayerPlan& p, const MoeLayerTypes& q, const MoeLayerTensors& w,
                             const float* x, float* out, void* workspace, hipStream_t s);
 

@@ -560,11 +560,11 @@ static int sub_rows(int64_t rb, int cols, int chunk, int tp) {
 }
 
 bool moe_plan(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, uint32_t qa, uint32_t qb,
-              MoePlan* plan, bool out_major) {
+              MoePlan* plan, bool out_major, bool tokens) {
   if (n_tok <= 0 || top_k <= 0 || top_k > kMoeMaxTopK || top_k > n_expert ||
       n_expert > kMoeMaxExperts || n_embd <= 0 || n_ff <= 0 || n_tok > kMoeMaxTokens)
     return false;
-  if (out_major) return moe_plan_out_major(n_tok, top_k, n_expert, n_embd, n_ff, qa, qb, plan);
+  if (out_major) return moe_plan_out_major(n_tok, top_k, n_expert, n_embd, n_ff, qa, qb, plan, tokens);
   if (!expert_shape_ok(qa, n_embd, n_ff) || !expert_shape_ok(qb, n_ff, n_embd)) return false;
   if (n_tok > kMoeMaxTokens || n_embd % 32 != 0) return false;
   // one thread per 32-column half unit of a row at least

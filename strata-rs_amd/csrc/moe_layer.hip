@@ -55,9 +55,9 @@ constexpr int kShMaxSplit = 8;  // shares of the shared expert's columns
 static size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
 bool moe_layer_plan(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, int n_ff_sh,
-                    const MoeLayerTypes& q, MoeLayerPlan* plan, bool out_major) {
+                    const MoeLayerTypes& q, MoeLayerPlan* plan, bool out_major, bool tokens, bool sh_tokens) {
   MoeLayerPlan p{};
-  if (!moe_plan(n_tok, top_k, n_expert, n_embd, n_ff, q.gate, q.down, &p.moe, out_major)) return false;
+  if (!moe_plan(n_tok, top_k, n_expert, n_embd, n_ff, q.gate, q.down, &p.moe, out_major, tokens)) return false;
   if (q.up != q.gate || n_ff_sh <= 0) return false;
   // the matvecs of the layer, at the shapes the gemv kernels take
   if (!gemv_shape_ok(q.router, n_expert, n_embd, 1) || !gemv_shape_ok(q.gate_sh, n_ff_sh, n_embd, 1) ||
@@ -80,7 +80,7 @@ bool moe_layer_plan(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, in
   p.o_d = take(sizeof(float) * T * n_embd);
   p.o_s = take(sizeof(float) * T);
   // the readings (q6 flags) of gate and up are looked at by the launch
-  p.sh_tok = n_tok > 8 && q.gate_sh == q.up_sh && tok_ok(q.gate_sh, n_ff_sh, n_embd) &&
+  p.sh_tok = sh_tokens && n_tok > 8 && q.gate_sh == q.up_sh && tok_ok(q.gate_sh, n_ff_sh, n_embd) &&
              tok_ok(q.down_sh, n_embd, n_ff_sh);
   if (p.sh_tok) {
     const TokPlan gu = tok_plan(n_ff_sh, 2, n_embd, n_tok, kChipCus, kShMaxSplit);

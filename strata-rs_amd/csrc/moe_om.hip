@@ -286,7 +286,7 @@ static int om_rows(int rows, int cols, int mats, int s_max) {
 }
 
 bool moe_plan_out_major(int n_tok, int top_k, int n_expert, int n_embd, int n_ff, uint32_t qa, uint32_t qb,
-                        MoePlan* plan) {
+                        MoePlan* plan, bool tokens) {
   // gate / up rows are n_embd wide, down rows n_ff: whole 64-column units
   // of whole blocks, and the staged vectors fit LDS
   if (!device_quant(qa) || !device_quant(qb)) return false;
@@ -304,7 +304,7 @@ bool moe_plan_out_major(int n_tok, int top_k, int n_expert, int n_embd, int n_ff
   p.rb_b = byte_size(qb, n_ff);
   const int pairs = n_tok * top_k;
   p.s_max = pairs < n_expert ? pairs : n_expert;
-  p.tok = moe_tok_group(p, qa, qb);
+  p.tok = tokens ? moe_tok_group(p, qa, qb) : 0;
   const int ip = p.tok ? p.tok : 2;  // an expert's pairs, ip to a work item
   p.z_max = (pairs + p.s_max * (ip - 1)) / ip;
   p.nch_a = p.nch_b = 1;  // whole dot products: one chunk each
