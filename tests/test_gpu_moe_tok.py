@@ -16,12 +16,13 @@ import strata_hip as H
 from conftest import STRICT_TOL, check_parity
 from strata_hip import synth as S
 from test_gpu_moe_om import OM, om_tensors, om_views, oracle_om, layer_om_tensors
+from test_gpu_moe_ws import two_token_bytes
 
 pytestmark = pytest.mark.gpu
 Q8_0, Q4_K, Q5_K, Q6_K, IQ4_XS = 8, 12, 13, 14, 23
 
 
-def moe_dev(quants, flags, mats, n_expert, n_embd, n_ff, logits, x, top_k, offset=0):
+def moe_dev(quants, flags, mats, n_expert, n_embd, n_ff, logits, x, top_k, offset=0, nb=None):
     """offset: floats between x's start and a 256-byte boundary."""
     import torch
     n_tok = x.shape[0]
@@ -30,7 +31,7 @@ def moe_dev(quants, flags, mats, n_expert, n_embd, n_ff, logits, x, top_k, offse
     xb = torch.zeros(x.size + offset, device="cuda")
     xb[offset:] = torch.from_numpy(x.reshape(-1)).cuda()
     out = torch.full((n_tok, n_embd), float("nan"), device="cuda")
-    nb = H.moe_workspace_bytes(n_tok, top_k, n_expert, n_embd, n_ff, quants[0], quants[2])
+    nb = nb or H.moe_workspace_bytes(n_tok, top_k, n_expert, n_embd, n_ff, quants[0], quants[2])
     ws = torch.full((nb,), 0xFF, dtype=torch.uint8, device="cuda")
     H.moe_ffn_dev(*[(q, OM | f, t.data_ptr()) for q, f, t in zip(quants, flags, dev)], n_expert, n_embd, n_ff,
                   tl.data_ptr(), n_tok, top_k, xb.data_ptr() + 4 * offset, out.data_ptr(), ws.data_ptr(), nb,
@@ -48,6 +49,9 @@ def moe_dev(quants, flags, mats, n_expert, n_embd, n_ff, logits, x, top_k, offse
     (Q8_0, Q8_0, 24, 1088, 320, 4, 16),   # rows of 34 and 10 blocks, one routing launch
     (IQ4_XS, Q4_K, 12, 256, 1024, 5, 17),
     (Q6_K, Q6_K, 32, 768, 2304, 2, 15),
+    (Q8_0, Q8_0, 24, 1088, 320, 4, 24),
+    (IQ4_XS, Q4_K, 12, 256, 1024, 5, 20),
+    (Q4_K, Q6_K, 32, 768, 1024, 4, 16),   # one routing launch
 ])
 def test_moe_many_tokens(oracle, qg, qd, n_expert, n_embd, n_ff, top_k, n_tok):
     print("[case] moe tokens", qg, qd, n_expert, n_embd, n_ff, top_k, n_tok, flush=True)
@@ -62,6 +66,30 @@ def test_moe_many_tokens(oracle, qg, qd, n_expert, n_embd, n_ff, top_k, n_tok):
         check_parity(got[t], want[t], f"token {t}")
     shifted = moe_dev((qg, qg, qd), (0, 0, 0), mats, n_expert, n_embd, n_ff, logits, x, top_k, offset=1)
     assert np.array_equal(got, shifted)
+
+
+# the many-token form is taken where it is the faster one: pairs x n_embd x
+# n_ff below and above the line of each kind of types, Q8_0 experts with fewer
+# and with more pairs than experts
+@pytest.mark.parametrize("qg,qd,n_expert,n_embd,n_ff,top_k,n_tok,tokens", [
+    (Q4_K, Q6_K, 32, 512, 1024, 2, 18, False), (Q4_K, Q6_K, 32, 512, 1024, 2, 20, True),
+    (Q5_K, Q5_K, 32, 512, 1024, 2, 20, False), (Q5_K, Q5_K, 32, 512, 1024, 2, 24, True),
+    (Q6_K, Q6_K, 32, 512, 1024, 2, 24, False), (Q6_K, Q6_K, 32, 512, 1024, 2, 29, True),
+    (Q8_0, Q4_K, 32, 512, 1024, 2, 24, False), (Q8_0, Q4_K, 32, 512, 1024, 2, 29, True),
+    (IQ4_XS, IQ4_XS, 16, 1536, 1024, 4, 8, False), (IQ4_XS, IQ4_XS, 16, 1536, 1024, 4, 11, True),
+    (Q8_0, Q8_0, 64, 512, 768, 8, 7, False), (Q8_0, Q8_0, 80, 1024, 1024, 8, 8, False),
+    (Q6_K, Q8_0, 80, 1024, 1024, 8, 8, False), (Q6_K, Q8_0, 64, 1024, 1024, 8, 8, True),
+])
+def test_moe_many_tokens_rule(qg, qd, n_expert, n_embd, n_ff, top_k, n_tok, tokens):
+    """A workspace of the two-token form's size always runs that form: the
+    call gives its bits with all of the workspace where the rule keeps it, and
+    other roundings where it does not."""
+    print("[case] moe tokens, rule", qg, qd, n_expert, n_embd, n_ff, top_k, n_tok, flush=True)
+    mats = om_tensors(n_expert, n_embd, n_ff, qg, qd, 65)
+    logits = S.router_logits(66, n_tok, n_expert)
+    x = S.normal_f32(67, n_tok * n_embd).reshape(n_tok, n_embd)
+    args = ((qg, qg, qd), (0, 0, 0), mats, n_expert, n_embd, n_ff, logits, x, top_k)
+    assert np.array_equal(moe_dev(*args), moe_dev(*args, nb=two_token_bytes(n_tok, top_k, n_expert, n_embd, n_ff))) != tokens
 
 
 def test_moe_all_tokens_on_the_same_experts(oracle):
