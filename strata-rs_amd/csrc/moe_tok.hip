@@ -33,24 +33,37 @@ static TokPlan moe_tok_plan(const MoePlan& p, int rows, int mats, int cols) {
 // 169 us in groups of 8, 217 of 16, 191 of 32; 256 tokens, average 16, 299, 302
 // and 214), or 0: moe_om.hip's launches, three fewer and one pass over the
 // weights per two pairs, stay the faster form for few pairs of small experts.
-// Where that ends depends on the types, as the two-token form costs the more
-// the more a weight's decode does. Both measured over five shapes from 12 to
-// 130 M of pairs x n_embd x n_ff, all 25 pairs of types; us, two-token form
-// and this one, 32 x 1024 x 512 top-2 at 24 tokens (25 M): Q4_K / Q6_K 34.6 /
-// 34.0, Q6_K / Q6_K 1.07 of it, Q8_0 / Q4_K 35.7 / 37.6; 64 x 1536 x 1024 top-4
-// at 8 (50 M): Q4_K / Q6_K 61.6 / 53.2, IQ4_XS / IQ4_XS 58.0 / 55.7 (with the
-// layer's other work beside it 84.4 / 90.1, 128 x 2048 x 768 top-8 at 5 IQ4_XS /
-// Q5_K 83 / 87). Q8_0 rows (limb dots) gain only
-// where experts are shared: 128 x 2048 x 768 top-8 at 8 tokens Q8_0 / Q8_0
-// 1.16, Q6_K / Q8_0 at 6 1.09, 32 x 1792 x 512 top-4 at 15 Q8_0 / Q8_0 0.99, at
-// 24 0.75. Far above the line, 128 x 2048 x 768 top-8 Q4_K / Q6_K: 16 tokens
-// 176 / 97, 96 640 / 183, 256 1465 / 214.
+// Where that ends depends on the types: the two-token form costs the more the
+// more a weight's decode does, and its limb dots of Q8_0 rows cost least. Both
+// measured over seven shapes from 12 to 130 M of pairs x n_embd x n_ff, all 25
+// pairs of types, this form's time over the two-token form's:
+//   32 x 1024 x 512 top-2, 24 tokens (25 M)  Q4_K / Q6_K 0.96, Q5_K / Q6_K
+//     1.00, Q6_K / Q6_K 1.07, Q8_0 / Q4_K 1.05; 31 tokens (33 M) 0.80, 0.82,
+//     0.87, 0.87
+//   64 x 1536 x 1024 top-4, 8 tokens (50 M)  Q4_K / Q6_K 0.85, IQ4_XS / IQ4_XS
+//     0.96, Q8_0 / Q5_K 1.02, Q8_0 / Q8_0 1.10; 6 tokens (38 M) 0.88, 1.04,
+//     1.07, 1.14
+// and, Q8_0 matrices only, on how many pairs an expert has:
+//   0.31 pairs an expert (128 experts, 5 tokens x 8)  Q5_K / Q8_0 1.03, Q6_K /
+//     Q8_0 1.06, Q8_0 / Q6_K 1.02, Q8_0 / Q8_0 1.15; 0.5 (8 tokens) 0.92,
+//     0.99, 1.02, 1.16; 0.69 (64 experts, 11 x 4) 0.72, 0.92, 0.84, 1.05;
+//     0.94 (15 x 4) 0.64, 0.85, 0.86, 0.99; 1.9 (32 experts, 15 x 4, 55 M)
+//     Q8_0 / Q4_K 0.83, Q8_0 / Q6_K 0.89
+// Far above the line, 128 x 2048 x 768 top-8 Q4_K / Q6_K, us: 16 tokens 176 /
+// 97, 96 640 / 183, 256 1465 / 214.
 int moe_tok_group(const MoePlan& p, uint32_t qa, uint32_t qb) {
   if (!tok_ok(qa, p.n_ff, p.n_embd) || !tok_ok(qb, p.n_embd, p.n_ff)) return 0;
   const int64_t pairs = int64_t(p.n_tok) * p.top_k, work = pairs * p.n_embd * p.n_ff;
-  const int64_t least = p.n_tok < 16 ? (qa == kIQ4_XS ? 65 : 50) : qa == kQ4_K ? 20 : qa == kQ6_K || qa == kQ8_0 ? 30 : 24;
+  const int64_t least = p.n_tok < 16 ? (qa == kQ8_0 && pairs < p.n_expert ? 60 : 50)
+                        : qa == kQ6_K || qa == kQ8_0 ? 30
+                        : qa == kQ4_K || qb == kQ4_K ? 20
+                                                     : 24;
   if (p.n_tok <= 4 || work < least * 1000000) return 0;
-  if ((qa == kQ8_0 || (qb == kQ8_0 && qa != kQ4_K)) && pairs < p.n_expert) return 0;
+  // eighths of a pair an expert
+  const int shared = qa == kQ8_0 ? (qb == kQ8_0 ? 6 : qb == kQ4_K || qb == kQ5_K ? 0 : 5)
+                     : qb == kQ8_0 ? (qa == kQ4_K ? 0 : qa == kQ6_K ? 5 : 3)
+                                   : 0;
+  if (8 * pairs < int64_t(shared) * p.n_expert) return 0;
   const int64_t avg = (pairs + p.s_max - 1) / p.s_max;
   return avg <= 8 ? 8 : avg <= 32 ? 32 : avg <= 64 ? 64 : 96;
 }

@@ -69,16 +69,20 @@ def test_moe_many_tokens(oracle, qg, qd, n_expert, n_embd, n_ff, top_k, n_tok):
 
 
 # the many-token form is taken where it is the faster one: pairs x n_embd x
-# n_ff below and above the line of each kind of types, Q8_0 experts with fewer
-# and with more pairs than experts
+# n_ff below and above the line of each kind of types, Q8_0 matrices with fewer
+# and with more pairs an expert
 @pytest.mark.parametrize("qg,qd,n_expert,n_embd,n_ff,top_k,n_tok,tokens", [
     (Q4_K, Q6_K, 32, 512, 1024, 2, 18, False), (Q4_K, Q6_K, 32, 512, 1024, 2, 20, True),
     (Q5_K, Q5_K, 32, 512, 1024, 2, 20, False), (Q5_K, Q5_K, 32, 512, 1024, 2, 24, True),
     (Q6_K, Q6_K, 32, 512, 1024, 2, 24, False), (Q6_K, Q6_K, 32, 512, 1024, 2, 29, True),
     (Q8_0, Q4_K, 32, 512, 1024, 2, 24, False), (Q8_0, Q4_K, 32, 512, 1024, 2, 29, True),
-    (IQ4_XS, IQ4_XS, 16, 1536, 1024, 4, 8, False), (IQ4_XS, IQ4_XS, 16, 1536, 1024, 4, 11, True),
-    (Q8_0, Q8_0, 64, 512, 768, 8, 7, False), (Q8_0, Q8_0, 80, 1024, 1024, 8, 8, False),
-    (Q6_K, Q8_0, 80, 1024, 1024, 8, 8, False), (Q6_K, Q8_0, 64, 1024, 1024, 8, 8, True),
+    (IQ4_XS, IQ4_XS, 16, 1536, 1024, 4, 7, False), (IQ4_XS, IQ4_XS, 16, 1536, 1024, 4, 8, True),
+    (Q8_0, Q5_K, 40, 1536, 1024, 4, 9, False), (Q8_0, Q5_K, 40, 1536, 1024, 4, 10, True),
+    (Q8_0, Q5_K, 16, 1536, 1024, 4, 8, True),
+    (Q8_0, Q8_0, 96, 1024, 1024, 8, 8, False), (Q8_0, Q8_0, 80, 1024, 1024, 8, 8, True),
+    (Q8_0, Q6_K, 112, 1024, 1024, 8, 8, False), (Q8_0, Q6_K, 96, 1024, 1024, 8, 8, True),
+    (Q6_K, Q8_0, 112, 1024, 1024, 8, 8, False), (Q6_K, Q8_0, 96, 1024, 1024, 8, 8, True),
+    (Q5_K, Q8_0, 96, 1536, 1024, 4, 8, False), (Q5_K, Q8_0, 80, 1536, 1024, 4, 8, True),
 ])
 def test_moe_many_tokens_rule(qg, qd, n_expert, n_embd, n_ff, top_k, n_tok, tokens):
     """A workspace of the two-token form's size always runs that form: the
