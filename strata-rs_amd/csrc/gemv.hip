@@ -1027,35 +1027,38 @@ static hipError_t launch_nb(int nb, const uint8_t* w, int rows, int cols, int64_
 }
 
 // Vectors per launch of gemv_q6win_kernel (as even as they go), 0: a shape it
-// does not take. It pays where it takes fewer rounds of waves: two rows a wave
-// against one, each of its rounds about 1.4 of gemv_kernel's (4096 x 6144, four
-// vectors, us before and now: 2048 rows, one round of either, 9.7 / 13.9; 4096,
-// two against one, 17.5 / 15.0; 6000, three against two, 22.4 / 22.8; 8192,
-// four against two, 27.1 / 22.7). It takes four vectors at most, so it needs no
-// more launches than gemv_kernel does, which takes eight where LDS holds them,
-// or so many rows that a launch more costs less than it saves (x 4096, us: 8192
-// rows, 8 vectors 29.2 / 27.9, 7 26.1 / 25.9, 6 23.6 / 24.4; 10240, half a
-// round left over, 8 34.4 / 36.3; 32768, 8 89.8 / 80.1, 7 79.7 / 76.2, 6 70.3
-// / 72.1; 65536, 6 131 / 121, 5 114 / 112). A vector by itself that
-// gemv_kernel leaves over takes the batch-1 form, which costs less than a pair
-// (8192 x 8192, 5 vectors as 4 + 1 40.0, as 3 + 2 40.9).
+// does not take. It pays where it takes fewer rounds of waves (two rows a wave
+// against one): its rounds take about 1.2 times gemv_kernel's at 2048 and 4096
+// columns and 1.4 above, where vectors leave LDS for one workgroup a CU.
+// Its time over gemv_kernel's, four vectors of 2048 / 4096 / 6144 columns:
+//   2048 rows, one round of either 1.19 / 1.25 / 1.42; 4096, two against one
+//   0.70 / 0.82 / 0.86; 6144, three against two 0.87 / 0.93 / 1.02; 8192, four
+//   against two 0.72 / 0.79 / 0.84; 9300, five against three 0.82 / 0.88 / 0.97
+// It holds four vectors at most, so it needs no more launches than gemv_kernel,
+// which takes eight where LDS holds them, or so many rows that a launch more
+// costs less than it saves (2048 / 4096 columns: 4096 rows, 8 vectors 0.90 /
+// 0.99, 7 0.95 / 1.04, 6 0.98 / 1.06; 10240, half a round left over, 8 1.00 /
+// 1.05; 17000, 8 0.76 / 0.87, 7 0.82 / 0.92, 6 0.89 / 0.98; 40000, 6 0.93 /
+// 0.97, 5 1.02 / 1.10). A vector by itself that gemv_kernel leaves over takes
+// the batch-1 form, which costs less than a pair (8192 x 8192, 5 vectors as 4
+// + 1 40.0 us, as 3 + 2 40.9).
 static size_t q6win_lds(int cols, int nb, int waves) {
   return size_t(nb) * xw_stride(cols) * sizeof(float) + size_t(waves) * 2 * kWinQ6;
 }
 static int q6win_batch(const uint8_t* w, int rows, int cols, int batch) {
   if (batch < 2 || cols % 2048 != 0 || (reinterpret_cast<uintptr_t>(w) & 15u)) return 0;
-  // rounds of gemv_kernel's waves (a sixteenth of a round does not count) and of this form's
-  const int64_t round = 8 * cu_count();
-  const int64_t one = (rows + round - round / 16 - 1) / round, two = (rows + 2 * round - 1) / (2 * round);
-  if (3 * two >= 2 * one) return 0;
+  // rounds of gemv_kernel's waves and of this form's
+  const int64_t round = 8 * cu_count(), one = (rows + round - 1) / round, two = (rows + 2 * round - 1) / (2 * round);
+  if (cols <= 4096 ? two >= one : 3 * two >= 2 * one) return 0;
   int most = 4;
   while (most >= 2 && q6win_lds(cols, most, 8) > kMaxLds) --most;
   if (most < 2) return 0;
   const int n = (batch + most - 1) / most, per = (batch + n - 1) / n;
   const int held = std::min(8, int(kMaxLds / lds_bytes(cols, 1))), before = (batch + held - 1) / held;
   if (n > before) {
-    const int64_t many = batch == 8 ? 4 : batch == 7 ? 16 : batch == 6 ? 32 : 1 << 30;
-    if (before > 1 || n > 2 || rows < many * round || 9 * two > 5 * one) return 0;
+    const bool narrow = cols <= 2048;
+    const int many = batch == 8 ? 1 : batch == 7 ? 8 : batch == 6 ? (narrow ? 9 : 16) : 1 << 30;  // rounds
+    if (before > 1 || n > 2 || one < many || (narrow ? 8 : 9) * two > 5 * one) return 0;
   }
   if (batch % held == 1 && 3 * n > batch) return 0;
   // (the last launch takes what is left, at least two)

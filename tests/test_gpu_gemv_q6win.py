@@ -47,10 +47,11 @@ def test_gemv_q6_windows(oracle, rows, cols, batch, offset, flags):
 # is taken where it is the faster one (rows a quarter round under the count)
 @pytest.mark.parametrize("rounds,cols,batch,windowed", [
     (1, 2048, 2, False), (1, 4096, 4, False), (1, 12288, 2, False),  # one round of either
-    (3, 2048, 2, False),                                            # two rounds against three
+    (3, 6144, 2, False), (3, 2048, 4, True),                        # two rounds against three
     (2, 2048, 5, False), (4, 4096, 6, False), (2, 8192, 4, False),  # a launch more
-    (5, 2048, 8, False), (4, 8192, 5, False),                       # half a round left over; a vector by itself
+    (5, 4096, 8, False), (4, 8192, 5, False),                       # half a round left over; a vector by itself
     (2, 2048, 2, True), (2, 4096, 4, True), (2, 8192, 3, True), (2, 6144, 6, True), (6, 2048, 8, True),
+    (2, 2048, 8, True), (9, 2048, 7, True),
 ])
 def test_gemv_q6_windows_rule(rounds, cols, batch, windowed):
     """gemv_kernel computes a row the same way wherever its weights start, and
