@@ -25,7 +25,8 @@
 // values themselves (fmt.hpp; their unsigned codes meet no such bias, and
 // f32 x keeps the full 24 bits that limbs round to 22 below each block's
 // maximum, which the silu(h) * p -> down -> weighted-sum chain amplifies
-// where experts cancel). A row's 64-column units
+// where experts cancel; the many-token form's f16 pairs, tok.hpp, hold 23
+// bits of each element by itself). A row's 64-column units
 // are spread over L lanes (L the power of two at or above the unit count, at
 // most 64), so 64 / L rows share a wave and narrow rows (a 768-wide down
 // input is 12 units) keep most lanes busy; the L lanes' sums are added with

@@ -2,11 +2,15 @@
 // precision (tok_mm.hip): the operand formats.
 //
 // Activations. Per 256-element super-block of a token a power of two 2^k
-// brings its largest |x| into [2^14, 2^15), and every x * 2^k is the sum of
-// two f16 numbers, hi = f16(x 2^k) and lo = f16(x 2^k - hi): 22 bits of each
-// element, whatever its size beside its neighbours (an f16 goes down to
-// 2^-24, 2^-39 of the maximum). Both enter v_mfma_f32_*_f16, whose products
-// are exact and whose sums are f32.
+// brings its largest |x| into [2^14, 2^15), and every y = x * 2^k is held as
+// hi + 2^-11 lo, hi = f16(y) and lo = f16(2^11 (y - hi)): y to within 2^-23 of
+// itself (a remainder has 12 bits and a sign, an f16 11: the last of the 24 is
+// lost in one element of four), whatever its size beside its neighbours down
+// to 2^-27 of the maximum, and below to within 2^-50 of that (lo's own scale
+// keeps it off f16's subnormals, where hi + lo would fall short from 2^-17 of
+// the maximum on). Both enter v_mfma_f32_*_f16, whose products are exact and
+// whose sums are f32; lo's factor 2^-11 is in the weights it meets (or, where
+// hi and lo are rows of one fragment, joins with the sums).
 // Weights. Codes become exact f16 integers: Q4_K / Q5_K codes times their
 // 6-bit sub-block scale (<= 63 * 31, 11 bits), the others the codes alone,
 // their sub-block scale applied to each sub-block's f32 sums. The block's d
@@ -66,6 +70,7 @@ __device__ __forceinline__ f16x2_t h2_dup(float v) {
 // A B fragment (the lane's 8 weights of one k step): word pairs hold bytes
 // (0, 2) and (1, 3) of a code word, so slot order within 4 columns is
 // 0, 2, 1, 3 (tok_slot); the activations are stored in the same order.
+constexpr float kTokLo = 0x1p-11f;  // of a lo limb
 union TokFrag {
   f16x2_t h[4];
   f16x8_t v;
@@ -89,7 +94,7 @@ __device__ __forceinline__ void tok_signed4(uint32_t w, f16x2_t& a, f16x2_t& b) 
 // 64 columns (32-column sub-blocks 2g and 2g + 1), each four MFMA k steps
 // (sub-block jj, step i). load<g> issues group g's loads into Raw; take<g>
 // moves what they brought into Sb (the next super-block's loads then go into
-// Raw); frags<g> forms the group's four B fragments, and sub<g> the
+// Raw); frags<g, jj> forms the two B fragments of sub-block jj, and sub<g> the
 // sub-block scales of the k steps (kSub 1) or sub-blocks (kSub 2). kSub 0:
 // the scales are in the weights. `left`: Q8_0 blocks from the super-block's
 // first to the row's last.
@@ -154,35 +159,26 @@ struct TokQ4Q5 {  // Q4_K, Q5_K
     v[7] = static_cast<_Float16>(ubyte<3>(m47));
     return v;
   }
-  template <int G>
-  __device__ static __forceinline__ void frags(const Sb& s, TokFrag (&f)[4]) {
-    const uint32_t sw = G < 2 ? s.sc03 : s.sc47;
-    const f16x2_t s0 = h2_dup((G & 1) ? ubyte<2>(sw) : ubyte<0>(sw)), s1 = h2_dup((G & 1) ? ubyte<3>(sw) : ubyte<1>(sw));
-    const f16x2_t c0 = s0 * h2_dup(-1024.f);
+  template <int G, int JJ>
+  __device__ static __forceinline__ void frags(const Sb& s, TokFrag (&f)[2]) {
+    const f16x2_t sc = h2_dup(ubyte<2 * (G & 1) + JJ>(G < 2 ? s.sc03 : s.sc47));
+    // Q4_K's high nibbles stay in place: 64 + q is the f16 with bits
+    // 0x5400 | q << 4
+    constexpr bool kHigh = Q != kQ5_K && JJ == 1;
+    const f16x2_t c = sc * h2_dup(kHigh ? -64.f : -1024.f);
     const uint32_t q[4] = {s.q.x, s.q.y, s.q.z, s.q.w};
-    if constexpr (Q == kQ5_K) {
-      const uint32_t qh[4] = {s.qh.x, s.qh.y, s.qh.z, s.qh.w};
-      const f16x2_t c1 = s1 * h2_dup(-1024.f);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        uint32_t lo, hi;
-        q5k_codes(q[k], qh[k], G, lo, hi);
-        tok_scaled4(lo, s0, c0, f[k >> 1].h[2 * (k & 1)], f[k >> 1].h[2 * (k & 1) + 1]);
-        tok_scaled4(hi, s1, c1, f[2 + (k >> 1)].h[2 * (k & 1)], f[2 + (k >> 1)].h[2 * (k & 1) + 1]);
-      }
-    } else {
-      // low nibbles as above; high nibbles stay in place: 64 + q is the f16
-      // with bits 0x5400 | q << 4
-      const f16x2_t c1 = s1 * h2_dup(-64.f);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t w = q[k], v = q[k] >> 8;
-        f16x2_t* lo = f[k >> 1].h + 2 * (k & 1);
-        f16x2_t* hi = f[2 + (k >> 1)].h + 2 * (k & 1);
-        lo[0] = __builtin_elementwise_fma(as_h2((w & 0x000F000Fu) | 0x64006400u), s0, c0);
-        lo[1] = __builtin_elementwise_fma(as_h2((v & 0x000F000Fu) | 0x64006400u), s0, c0);
-        hi[0] = __builtin_elementwise_fma(as_h2((w & 0x00F000F0u) | 0x54005400u), s1, c1);
-        hi[1] = __builtin_elementwise_fma(as_h2((v & 0x00F000F0u) | 0x54005400u), s1, c1);
+    for (int k = 0; k < 4; ++k) {
+      f16x2_t* o = f[k >> 1].h + 2 * (k & 1);
+      if constexpr (Q == kQ5_K) {
+        const uint32_t qh[4] = {s.qh.x, s.qh.y, s.qh.z, s.qh.w};
+        uint32_t code[2];
+        q5k_codes(q[k], qh[k], G, code[0], code[1]);
+        tok_scaled4(code[JJ], sc, c, o[0], o[1]);
+      } else {
+        constexpr uint32_t kMask = kHigh ? 0x00F000F0u : 0x000F000Fu, kBits = kHigh ? 0x54005400u : 0x64006400u;
+        o[0] = __builtin_elementwise_fma(as_h2((q[k] & kMask) | kBits), sc, c);
+        o[1] = __builtin_elementwise_fma(as_h2(((q[k] >> 8) & kMask) | kBits), sc, c);
       }
     }
   }
@@ -256,25 +252,26 @@ struct TokQ6 {
       s.ql[1] = halves(win16(r.ql[G + 1], r.sh));
     }
   }
-  template <int G>
-  __device__ static __forceinline__ void frags(const Sb& s, TokFrag (&f)[4]) {
+  template <int G, int JJ>
+  __device__ static __forceinline__ void frags(const Sb& s, TokFrag (&f)[2]) {
     const f16x2_t bias = as_h2(0xE420E420u);  // -(1024 + 32)
+    // 32-column group I = 2 (G & 1) + JJ of the half: ql run JJ, nibble G & 1,
+    // bit pair I of qh
+    constexpr int I = 2 * (G & 1) + JJ;
+    const uint32_t q[4] = {s.ql[JJ].x, s.ql[JJ].y, s.ql[JJ].z, s.ql[JJ].w};
+    const uint32_t qh[4] = {s.qh.x, s.qh.y, s.qh.z, s.qh.w};
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      // 32-column group i' = 2 (G & 1) + jj of the half: ql run jj, nibble
-      // G & 1, bit pair i' of qh
-      const uint32_t q[4] = {s.ql[jj].x, s.ql[jj].y, s.ql[jj].z, s.ql[jj].w};
-      const uint32_t qh[4] = {s.qh.x, s.qh.y, s.qh.z, s.qh.w};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t lo = (G & 1) ? (q[k] >> 4) & 0x0F0F0F0Fu : q[k] & 0x0F0F0F0Fu;
-        constexpr int P = 2 * (G & 1);
-        const uint32_t t = (P + jj) < 2 ? qh[k] << (4 - 2 * (P + jj)) : qh[k] >> (2 * (P + jj) - 4);
-        const uint32_t w = lo | (t & 0x30303030u);
-        f16x2_t* o = f[2 * jj + (k >> 1)].h + 2 * (k & 1);
-        o[0] = as_h2((w & 0x003F003Fu) | 0x64006400u) + bias;
-        o[1] = as_h2(((w >> 8) & 0x003F003Fu) | 0x64006400u) + bias;
-      }
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t lo = (G & 1) ? (q[k] >> 4) & 0x0F0F0F0Fu : q[k] & 0x0F0F0F0Fu;
+      uint32_t t;
+      if constexpr (I < 2)
+        t = qh[k] << (4 - 2 * I);
+      else
+        t = qh[k] >> (2 * I - 4);
+      const uint32_t w = lo | (t & 0x30303030u);
+      f16x2_t* o = f[k >> 1].h + 2 * (k & 1);
+      o[0] = as_h2((w & 0x003F003Fu) | 0x64006400u) + bias;
+      o[1] = as_h2(((w >> 8) & 0x003F003Fu) | 0x64006400u) + bias;
     }
   }
   template <int G>
@@ -337,16 +334,13 @@ struct TokQ8 {
     }
   }
   __device__ static __forceinline__ float d(const Sb&) { return 1.f; }
-  template <int G>
-  __device__ static __forceinline__ void frags(const Sb& s, TokFrag (&f)[4]) {
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const u32x4 q = s.q[jj];
-      tok_signed4(q.x, f[2 * jj].h[0], f[2 * jj].h[1]);
-      tok_signed4(q.y, f[2 * jj].h[2], f[2 * jj].h[3]);
-      tok_signed4(q.z, f[2 * jj + 1].h[0], f[2 * jj + 1].h[1]);
-      tok_signed4(q.w, f[2 * jj + 1].h[2], f[2 * jj + 1].h[3]);
-    }
+  template <int G, int JJ>
+  __device__ static __forceinline__ void frags(const Sb& s, TokFrag (&f)[2]) {
+    const u32x4 q = s.q[JJ];
+    tok_signed4(q.x, f[0].h[0], f[0].h[1]);
+    tok_signed4(q.y, f[0].h[2], f[0].h[3]);
+    tok_signed4(q.z, f[1].h[0], f[1].h[1]);
+    tok_signed4(q.w, f[1].h[2], f[1].h[3]);
   }
   template <int G>
   __device__ static __forceinline__ void sub(const Sb& s, float (&sc)[4], int, int left) {
@@ -386,16 +380,13 @@ struct TokIQ4 {
     }
   }
   __device__ static __forceinline__ float d(const Sb& s) { return h2f(s.h.x); }
-  template <int G>
-  __device__ static __forceinline__ void frags(const Sb& s, TokFrag (&f)[4]) {
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const u32x2 q = s.q[jj];
-      tok_signed4(iq4_lut(q.x & 0x0F0F0F0Fu), f[2 * jj].h[0], f[2 * jj].h[1]);
-      tok_signed4(iq4_lut(q.y & 0x0F0F0F0Fu), f[2 * jj].h[2], f[2 * jj].h[3]);
-      tok_signed4(iq4_lut((q.x >> 4) & 0x0F0F0F0Fu), f[2 * jj + 1].h[0], f[2 * jj + 1].h[1]);
-      tok_signed4(iq4_lut((q.y >> 4) & 0x0F0F0F0Fu), f[2 * jj + 1].h[2], f[2 * jj + 1].h[3]);
-    }
+  template <int G, int JJ>
+  __device__ static __forceinline__ void frags(const Sb& s, TokFrag (&f)[2]) {
+    const u32x2 q = s.q[JJ];
+    tok_signed4(iq4_lut(q.x & 0x0F0F0F0Fu), f[0].h[0], f[0].h[1]);
+    tok_signed4(iq4_lut(q.y & 0x0F0F0F0Fu), f[0].h[2], f[0].h[3]);
+    tok_signed4(iq4_lut((q.x >> 4) & 0x0F0F0F0Fu), f[1].h[0], f[1].h[1]);
+    tok_signed4(iq4_lut((q.y >> 4) & 0x0F0F0F0Fu), f[1].h[2], f[1].h[3]);
   }
   template <int G>
   __device__ static __forceinline__ void sub(const Sb& s, float (&sc)[4], int, int) {

@@ -14,11 +14,12 @@
 // per token group, a super-block ahead; the group's A fragments come
 // through a ring of three LDS buffers (global_load_lds, two stages ahead)
 // that the four waves share. A group is
-//   32, 64 or 96 tokens: hi and lo limbs are fragments of their own, both
-//     added into the same f32 sums (a stage is 64 columns);
+//   32, 64 or 96 tokens: hi and lo limbs are fragments of their own, lo's
+//     against 2^-11 of the weights into hi's f32 sums or, where registers
+//     allow, into sums of their own (a stage is 64 columns);
 //   8 or 16 tokens: the hi limbs are A rows [0, T) and the lo limbs rows
-//     [T, 2 T) of one fragment, so no matrix work is done for padding at 16
-//     (a stage is a whole super-block).
+//     [T, 2 T) of one fragment, so no matrix work is done for padding at 16,
+//     and their sums are added at the end (a stage is a whole super-block).
 // Bound: weights are read and decoded once per group, so few tokens are
 // bound by the weight stream and many by MFMA (two f16 products per weight
 // and token). Per launch in a kernel trace: gate and up of 4096 x 12288 Q4_K
@@ -131,10 +132,11 @@ __global__ void __launch_bounds__(256) tok_prep_kernel(TokPrep a) {
   h01[1] = static_cast<_Float16>(y2);
   h23[0] = static_cast<_Float16>(y1);
   h23[1] = static_cast<_Float16>(y3);
-  l01[0] = static_cast<_Float16>(y0 - static_cast<float>(h01[0]));
-  l01[1] = static_cast<_Float16>(y2 - static_cast<float>(h01[1]));
-  l23[0] = static_cast<_Float16>(y1 - static_cast<float>(h23[0]));
-  l23[1] = static_cast<_Float16>(y3 - static_cast<float>(h23[1]));
+  auto low = [](float y, _Float16 h) { return static_cast<_Float16>((y - static_cast<float>(h)) * (1.f / kTokLo)); };
+  l01[0] = low(y0, h01[0]);
+  l01[1] = low(y2, h01[1]);
+  l23[0] = low(y1, h23[0]);
+  l23[1] = low(y3, h23[1]);
 
   const int j = lane >> 3, c = (4 * lane) & 31;  // sub-block, column in it
   const int i = a.perm ? c >> 4 : (c >> 3) & 1, half = a.perm ? (c >> 3) & 1 : c >> 4;
@@ -149,11 +151,12 @@ __global__ void __launch_bounds__(256) tok_prep_kernel(TokPrep a) {
     *reinterpret_cast<u32x2*>(p + piece + tok_row_byte(tok, row, half)) = lo;
 
   // sub-block sums of x as hi and lo of sum * 2^(k - 5), against the mins in
-  // both lane halves: apart in the k slots, or (packed) in the A rows
+  // both lane halves (lo's times 2^-11): apart in the k slots, or (packed) in
+  // the A rows
   uint8_t* sums = base + 4 * gbytes + tile * piece;
   if ((lane & 7) == 0) {
     const float y = ldexpf(s, k - 5);
-    const _Float16 sh = static_cast<_Float16>(y), sl = static_cast<_Float16>(y - static_cast<float>(sh));
+    const _Float16 sh = static_cast<_Float16>(y), sl = low(y, sh);
     *reinterpret_cast<_Float16*>(sums + tok_row_byte(tok, row, 0) + 2 * j) = sh;
     if (packed) {
       *reinterpret_cast<_Float16*>(sums + tok_row_byte(tok, row + tok, 0) + 2 * j) = sl;
@@ -266,6 +269,12 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
   using S = TokShape<TOK>;
   constexpr int NT = S::kTiles;
   constexpr int kAcc = TOK == 8 ? 8 : 16;  // D values of a tile that are used
+  // lo limbs into sums of their own, up to 64 tokens where a super-block's
+  // sums stay in the MFMA's accumulators: fewer instructions than 2^-11 of
+  // every weight (4096 / 12288 Q4_K, 24 tokens: 58.0 us, else 59.4; lo on hi's
+  // own scale, short of bits beside large neighbours, 57.2)
+  constexpr bool kOwnLo = F::kSub == 0 && !S::kPacked && NT <= 2;
+  constexpr int kSums = kOwnLo ? 2 * NT : NT;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   const int r32 = lane & 31, half = lane >> 5;
@@ -317,24 +326,42 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
 
   // one 64-column group: its k steps into acc (kSub 0, over the super-block)
   // or scaled by sub-block into acc
-  auto group_mma = [&](auto G, const uint8_t* A, f32x16_t (&acc)[NT], int left) {
+  auto group_mma = [&](auto G, const uint8_t* A, f32x16_t (&acc)[kSums], int left) {
     constexpr int g = decltype(G)::value;
-    TokFrag f[4];
-    F::template frags<g>(sb, f);
+    // fragments of one sub-block at a time, or (32-column scales) of both
+    constexpr bool kBoth = F::kSub == 2;
+    TokFrag f[2][2];
+    auto frags = [&](int jj) {
+      if (jj == 0)
+        F::template frags<g, 0>(sb, f[0]);
+      else
+        F::template frags<g, 1>(sb, f[kBoth]);
+    };
     float sc[4];
     F::template sub<g>(sb, sc, a.q6s, left);
     auto frag_a = [&](int t, int k, int limb) {
       const int at = TOK == 8 ? (16 * half + (lane & 15)) * 16 : 16 * lane;
       return *reinterpret_cast<const f16x8_t*>(A + ((t * 4 + k) * S::kLimbs + limb) * S::kPiece + at);
     };
+    // the weights of k step k that a limb meets: integers up to 2^11, so
+    // 2^-11 of them is exact
+    auto frag_b = [&](int k, int limb) {
+      const f16x8_t w = f[kBoth ? k >> 1 : 0][k & 1].v;
+      return limb && !kOwnLo ? w * static_cast<_Float16>(kTokLo) : w;
+    };
     if constexpr (F::kSub == 0) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < 4; ++k) {
+        if (k % 2 == 0) frags(k / 2);
 #pragma unroll
         for (int limb = 0; limb < S::kLimbs; ++limb)
 #pragma unroll
           for (int t = 0; t < NT; ++t)
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag_a(t, k, limb), f[k].v, acc[t], 0, 0, 0);
+          {
+            f32x16_t& d = acc[kOwnLo && limb ? NT + t : t];
+            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag_a(t, k, limb), frag_b(k, limb), d, 0, 0, 0);
+          }
+      }
     } else {
       // unit u = (k steps of a sub-block, tile): its MFMAs go out before unit
       // u - 1's sums are scaled, so the two overlap and only two units' sums
@@ -345,12 +372,16 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
       for (int u = 0; u <= kUnits; ++u) {
         if (u < kUnits) {
           const int k = u / NT * kSteps, t = u % NT;
+          if (t == 0 && (kBoth ? k == 0 : k % 2 == 0)) {
+            frags(k / 2);
+            if constexpr (kBoth) frags(1);
+          }
           f32x16_t v = {};
 #pragma unroll
           for (int k2 = 0; k2 < kSteps; ++k2)
 #pragma unroll
             for (int limb = 0; limb < S::kLimbs; ++limb)
-              v = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag_a(t, k + k2, limb), f[k + k2].v, v, 0, 0, 0);
+              v = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag_a(t, k + k2, limb), frag_b(k + k2, limb), v, 0, 0, 0);
           dd[u & 1] = v;
         }
         if (u > 0) {
@@ -364,7 +395,7 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
     }
   };
   // a super-block's sums into y: y += 2^-k (d acc - dmin 2^5 mn)
-  auto finish_sb = [&](const uint8_t* sums, f32x16_t (&acc)[NT]) {
+  auto finish_sb = [&](const uint8_t* sums, f32x16_t (&acc)[kSums]) {
     const float d = F::d(sb);
     const float* pk = reinterpret_cast<const float*>(sums + S::kSums);
 #pragma unroll
@@ -374,8 +405,9 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
       if constexpr (F::kMin) {
         dm = -32.f * F::dmin(sb);
         const int at = TOK == 8 ? (16 * half + (lane & 15)) * 16 : 16 * lane;
+        const _Float16 lo = static_cast<_Float16>(!S::kPacked && half ? kTokLo : 1.f);
         mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const f16x8_t*>(sums + t * S::kPiece + at),
-                                                    F::mins(sb), mn, 0, 0, 0);
+                                                    F::mins(sb) * lo, mn, 0, 0, 0);
       }
 #pragma unroll
       for (int i4 = 0; i4 < kAcc / 4; ++i4) {
@@ -383,7 +415,9 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
         const f32x4 p = *reinterpret_cast<const f32x4*>(pk + tk);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          float v = d * acc[t][4 * i4 + i];
+          float v = acc[t][4 * i4 + i];
+          if constexpr (kOwnLo) v = __builtin_fmaf(kTokLo, acc[NT + t][4 * i4 + i], v);
+          v *= d;
           if constexpr (F::kMin) v = __builtin_fmaf(dm, mn[4 * i4 + i], v);
           y[t][4 * i4 + i] = __builtin_fmaf(p[i], v, y[t][4 * i4 + i]);
         }
@@ -448,7 +482,7 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
       stage(s + 2, slot == 0 ? 2 : slot - 1);
       const uint8_t* A = lds + slot * S::kSb;
       const int left = blk0 - 8 * s;
-      f32x16_t acc[NT] = {};
+      f32x16_t acc[kSums] = {};
       take(g0, cur);
       group_mma(g0, A, acc, left);
       take(g1, cur);
@@ -488,7 +522,7 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
     wait_vmem<kCopies>();
     int slot = 0;
     auto super_block = [&](int s, Raw& cur, Raw& next) {
-      f32x16_t acc[NT] = {};
+      f32x16_t acc[kSums] = {};
       const int left = blk0 - 8 * s;
       auto step = [&](auto G) {
         constexpr int g = decltype(G)::value;
@@ -532,7 +566,7 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
 #pragma unroll
     for (int i = 0; i < TOK / 2; ++i) {
       const int t = TOK == 8 ? 4 * half + i : 8 * (i >> 2) + 4 * half + (i & 3);
-      if (t < cnt) o[int64_t(t) * a.ld] = y[0][i] + y[0][i + TOK / 2];
+      if (t < cnt) o[int64_t(t) * a.ld] = __builtin_fmaf(kTokLo, y[0][i + TOK / 2], y[0][i]);
     }
   } else {
 #pragma unroll

@@ -6,7 +6,7 @@ rows that end inside a 256-column step (odd block counts included), weights
 at 2-byte alignment, every format in each of its readings.
 
 Tolerance: the matvec bars (conftest.check_parity) on out - x. The
-activations are held to 22 bits and every sum is f32, so the result is within
+activations are held to 23 bits and every sum is f32, so the result is within
 a few f32 roundings of the oracle's, as the 8-token matvecs are.
 """
 import numpy as np
@@ -85,6 +85,35 @@ def test_ffn_many_tokens_other_reading(oracle, quant, flag):
     got = ffn((quant,) * 3, (flag,) * 3, mats, n_embd, n_ff, x, norm)
     want = oracle.dense_ffn((0, 0, 0), [w.view(np.uint8) for w in f32], n_embd, n_ff, x, norm, 1e-6)
     check_parity(got.astype(np.float64) - x, want.astype(np.float64) - x, "ffn out - x")
+
+
+@pytest.mark.parametrize("n_tok", [12, 30, 60, 96])
+@pytest.mark.parametrize("quant", [Q8_0, Q6_K])
+def test_ffn_small_elements_beside_large_ones(oracle, quant, n_tok):
+    """Every element keeps its own bits: one column of each super-block is
+    2^28 times the others (its norm weight) and meets weights of 0, so the
+    outputs are the other columns'. They are held to 2^-22 of themselves there
+    (2^-50 of the maximum), through two products and f32 sums: 1e-5 of the
+    largest output (1.2e-6 and less where the sums are exact to f32; limbs that
+    end 2^-39 below the maximum give 1e-4)."""
+    print("[case] ffn tokens, small beside large", quant, n_tok, flush=True)
+    n_embd, n_ff = 768, 512
+    mats = [S.matrix(quant, 21, n_ff, n_embd), S.matrix(quant, 22, n_ff, n_embd), S.matrix(quant, 23, n_embd, n_ff)]
+    big = np.arange(3) * 256 + 5
+    for i in (0, 1):
+        if quant == Q8_0:  # block 0 of each eight: [d][32 codes]
+            b = mats[i].reshape(n_ff, n_embd // 256, 8, 34)
+            b[:, :, 0, 2 + 5] = 0
+        else:  # [ql 128][qh 64][sc 16][d]: code 32 in element 5
+            b = mats[i].reshape(n_ff, n_embd // 256, 210)
+            b[:, :, 5] &= 0xF0
+            b[:, :, 128 + 5] = (b[:, :, 128 + 5] & 0xFC) | 2
+    x = S.normal_f32(24 + n_tok, n_tok * n_embd).reshape(n_tok, n_embd)
+    norm = S.normal_f32(25, n_embd)
+    norm[big] = 2.0 ** 28
+    got = ffn((quant,) * 3, (0, 0, 0), mats, n_embd, n_ff, x, norm)
+    want = oracle.dense_ffn((quant,) * 3, mats, n_embd, n_ff, x, norm, 1e-6)
+    check_parity(got.astype(np.float64) - x, want.astype(np.float64) - x, "ffn out - x", norm_tol=1e-5, strict_tol=None)
 
 
 def test_ffn_workspace_of_more_tokens(oracle):
