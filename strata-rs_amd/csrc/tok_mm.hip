@@ -1,6 +1,7 @@
 // Weight rows against many token vectors: y[t][r] = sum_c W[r][c] x[t][c]
 // as `tokens` calls of ops::gemv (crates/strata-core/src/ops.rs:14-28), for
-// 2 tokens to thousands, at the matvecs' precision (tok.hpp's operands).
+// 9 tokens to thousands and for an expert's, at the matvecs' precision
+// (tok.hpp's operands).
 //
 // The launches: tok_prep_kernel converts the tokens once per call into the
 // MFMA's A fragments (a super-block of a token group is one contiguous run,
@@ -601,9 +602,7 @@ bool tok_ok(uint32_t quant, int64_t rows, int64_t cols) {
 
 TokPlan tok_plan(int64_t rows, int mats, int64_t cols, int tokens, int cu, int max_split) {
   TokPlan p{};
-  if (tokens <= 8) {
-    p.tok = 8;
-  } else if (tokens <= 16) {
+  if (tokens <= 16) {  // (fewer than 9 stay with the matvecs)
     p.tok = 16;
   } else {
     const int g = (tokens + 95) / 96;
@@ -612,8 +611,10 @@ TokPlan tok_plan(int64_t rows, int mats, int64_t cols, int tokens, int cu, int m
   p.groups = (tokens + p.tok - 1) / p.tok;
   p.nsb = int((cols + 255) / 256);
   p.tiles = int((rows + kTokRows - 1) / kTokRows) * mats;
-  // workgroups the chip holds at once: two per CU (LDS) from 64 tokens,
-  // about four below
+  // workgroups a round: two per CU (what LDS holds) from 64 tokens. Below it
+  // holds one to three with the weights' slots, and four are counted: fewer,
+  // longer shares took up to 9% more (three matrices of 5120 / 17408 Q6_K, 17
+  // tokens 124 us, counting two 135; 3584 / 8192, 9 tokens, 58 / 56)
   const int64_t slots = int64_t(cu) * (p.tok >= 64 ? 2 : 4);
   // shares of the columns: the fewest rounds of workgroups, each round as
   // long as a share plus about two super-blocks of start and end
