@@ -17,10 +17,11 @@ Q6_K = 14
 
 
 @pytest.mark.parametrize("rows,cols,batch,offset", [
-    (1, 2048, 2, 0), (17, 4096, 3, 0), (33, 6144, 4, 0), (40, 12288, 5, 0), (255, 2048, 6, 0), (64, 4096, 7, 0),
+    (2049, 2048, 2, 0), (2307, 4096, 3, 0), (3001, 6144, 4, 0), (2306, 12288, 6, 0), (2305, 6144, 7, 0),
     (13000, 2048, 8, 0),           # 12 waves a workgroup, rows past one round
-    (2305, 2048, 2, 0), (2307, 4096, 3, 0), (3001, 6144, 4, 0), (2306, 12288, 6, 0), (2305, 6144, 7, 0),
-    (31, 4096, 4, 2), (31, 4352, 4, 0),  # weights off 16 bytes, columns off 2048
+    # gemv_kernel: one round of rows, weights off 16 bytes, columns off 2048
+    (1, 2048, 2, 0), (17, 4096, 3, 0), (33, 6144, 4, 0), (40, 12288, 5, 0), (255, 2048, 6, 0), (64, 4096, 7, 0),
+    (31, 4096, 4, 2), (31, 4352, 4, 0),
 ])
 @pytest.mark.parametrize("flags", [0, H.FLAG_Q6K_SIGNED_SCALES])
 def test_gemv_q6_windows(oracle, rows, cols, batch, offset, flags):

@@ -34,6 +34,25 @@ def test_route_matches_oracle(backend, oracle, n_tok, n_expert, top_k):
         assert abs(float(w[t].astype(np.float64).sum()) - 1.0) < 1e-5
 
 
+@pytest.mark.parametrize("n_tok", [17, 256])
+@pytest.mark.parametrize("n_expert,top_k", [(64, 8), (65, 8), (128, 32), (200, 1), (500, 10), (1000, 32)])
+def test_route_many_tokens(backend, oracle, n_tok, n_expert, top_k):
+    """Above 16 tokens the routing is two launches (a wave a token, four tokens
+    a workgroup, then the grouping): every count of experts a lane, a last
+    workgroup partly filled, the most pairs, and tied logits."""
+    say("route, many tokens", n_tok, n_expert, top_k)
+    logits = S.router_logits(200 + n_tok + n_expert, n_tok, n_expert)
+    logits[3] = 0.0
+    logits[5] = np.round(logits[5])
+    logits[n_tok - 1, : n_expert // 2] = 1.0
+    ids, w = backend.moe_route(logits, top_k)
+    for t in range(n_tok):
+        oid, ow = oracle.moe_route(logits[t], top_k)
+        assert ids[t].tolist() == oid.tolist()
+        assert np.abs(w[t] - ow).max() <= 4e-7
+        assert abs(float(w[t].astype(np.float64).sum()) - 1.0) < 1e-5
+
+
 def test_route_ties_and_uniform(backend, oracle):
     say("route ties")
     lg = np.zeros((2, 16), np.float32)
@@ -63,6 +82,28 @@ def oracle_moe(oracle, qg, qd, n_expert, n_embd, n_ff, gate, up, down, logits, x
 def moe_config_tensors():
     # 128 experts, hidden 2048, expert intermediate 768 (about 26 s to synthesise)
     return expert_tensors(128, 2048, 768, 12, 14, 4000)
+
+
+@pytest.mark.parametrize("qg,qd,n_expert,n_embd,n_ff,top_k,n_tok", [
+    (12, 14, 128, 512, 256, 8, 17), (8, 13, 200, 256, 256, 4, 33), (13, 12, 65, 256, 512, 2, 256)])
+def test_moe_ffn_many_tokens(backend, oracle, qg, qd, n_expert, n_embd, n_ff, top_k, n_tok):
+    """In-major stacks above 16 tokens: the items of two tokens and the pairs'
+    places from ids that another launch routed."""
+    say("moe ffn, many tokens", qg, qd, n_expert, n_tok)
+    gate, up, down = expert_tensors(n_expert, n_embd, n_ff, qg, qd, 400 + n_tok)
+    logits = S.router_logits(401 + n_tok, n_tok, n_expert)
+    logits[2] = 0.0
+    x = S.normal_f32(402 + n_tok, n_tok * n_embd).reshape(n_tok, n_embd)
+    name = f"many{n_expert}"
+    views = (H.ExpertView(f"{name}.g", qg, n_expert, n_embd, n_ff, gate),
+             H.ExpertView(f"{name}.u", qg, n_expert, n_embd, n_ff, up),
+             H.ExpertView(f"{name}.d", qd, n_expert, n_ff, n_embd, down))
+    out = backend.moe_ffn(*views, logits, x, top_k)
+    ref = oracle_moe(oracle, qg, qd, n_expert, n_embd, n_ff, gate, up, down, logits, x, top_k)
+    for t in range(n_tok):
+        check_parity(out[t], ref[t], f"token {t}")
+    for v in views:
+        backend.evict(v.name)
 
 
 @pytest.mark.parametrize("n_tok", [1, 16])

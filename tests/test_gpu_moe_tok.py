@@ -5,15 +5,13 @@ on the same experts, rows that are no multiple of the 128-row tiles, every
 type, both routing forms (above and at 16 tokens), the shared expert in the
 whole layer, gate and up in two Q6_K readings, and x at float alignment.
 
-Bars: conftest.check_parity's, a token at a time, as the two-token form's;
-twice the per-element one where the reference is the device's own few-token
-form, itself within one bar of the oracle.
+Bars: conftest.check_parity's, a token at a time, as the two-token form's.
 """
 import numpy as np
 import pytest
 
 import strata_hip as H
-from conftest import STRICT_TOL, check_parity
+from conftest import check_parity
 from strata_hip import synth as S
 from test_gpu_moe_om import OM, om_tensors, om_views, oracle_om, layer_om_tensors
 from test_gpu_moe_ws import two_token_bytes
@@ -40,20 +38,31 @@ def moe_dev(quants, flags, mats, n_expert, n_embd, n_ff, logits, x, top_k, offse
     return out.cpu().numpy()
 
 
-@pytest.mark.parametrize("qg,qd,n_expert,n_embd,n_ff,top_k,n_tok", [
-    (Q4_K, Q6_K, 64, 512, 512, 4, 20),    # groups of 8
-    (Q5_K, Q4_K, 16, 512, 768, 6, 20),    # 8, most experts full
-    (Q6_K, Q8_0, 8, 1024, 256, 3, 40),    # 32
-    (Q8_0, Q5_K, 4, 512, 768, 2, 60),     # 64
-    (Q4_K, Q6_K, 3, 768, 512, 2, 90),     # 96
-    (Q8_0, Q8_0, 24, 1088, 320, 4, 16),   # rows of 34 and 10 blocks, one routing launch
-    (IQ4_XS, Q4_K, 12, 256, 1024, 5, 17),
-    (Q6_K, Q6_K, 32, 768, 2304, 2, 15),
-    (Q8_0, Q8_0, 24, 1088, 320, 4, 24),
-    (IQ4_XS, Q4_K, 12, 256, 1024, 5, 20),
-    (Q4_K, Q6_K, 32, 768, 1024, 4, 16),   # one routing launch
+def group(n_expert, top_k, n_tok):
+    """Tokens of an expert that share a pass over its weights (moe_tok_group)."""
+    pairs = n_tok * top_k
+    avg = -(-pairs // min(pairs, n_expert))
+    return next(g for g, most in ((8, 8), (32, 32), (64, 64), (96, pairs)) if avg <= most)
+
+
+@pytest.mark.parametrize("qg,qd,n_expert,n_embd,n_ff,top_k,n_tok,tokens", [
+    (Q4_K, Q6_K, 64, 512, 512, 4, 20, 8),
+    (Q5_K, Q4_K, 16, 512, 768, 6, 20, 8),     # most groups full
+    (Q6_K, Q8_0, 8, 1024, 256, 3, 40, 32),
+    (Q8_0, Q5_K, 4, 512, 768, 2, 60, 32),     # run over
+    (Q4_K, Q6_K, 3, 768, 512, 2, 90, 64),
+    (Q5_K, Q8_0, 3, 768, 512, 2, 110, 96),
+    (Q6_K, Q4_K, 2, 512, 768, 2, 110, 96),    # run over: 110 pairs an expert
+    (IQ4_XS, IQ4_XS, 2, 512, 768, 2, 97, 96),
+    (Q8_0, Q8_0, 3, 1088, 320, 2, 130, 96),   # rows of 34 and 10 blocks
+    (Q8_0, Q8_0, 24, 1088, 320, 4, 24, 8),
+    (IQ4_XS, Q4_K, 12, 256, 1024, 5, 17, 8),
+    (Q6_K, Q6_K, 32, 768, 2304, 2, 15, 8),
+    (Q4_K, Q6_K, 32, 768, 1024, 4, 16, 8),    # one routing launch
+    (Q8_0, Q8_0, 24, 1088, 320, 4, 16, 0),    # stays with the two-token form
 ])
-def test_moe_many_tokens(oracle, qg, qd, n_expert, n_embd, n_ff, top_k, n_tok):
+def test_moe_many_tokens(oracle, qg, qd, n_expert, n_embd, n_ff, top_k, n_tok, tokens):
+    assert tokens in (0, group(n_expert, top_k, n_tok))
     print("[case] moe tokens", qg, qd, n_expert, n_embd, n_ff, top_k, n_tok, flush=True)
     mats = om_tensors(n_expert, n_embd, n_ff, qg, qd, 60 + n_tok)
     logits = S.router_logits(61 + n_tok, n_tok, n_expert)
@@ -66,6 +75,10 @@ def test_moe_many_tokens(oracle, qg, qd, n_expert, n_embd, n_ff, top_k, n_tok):
         check_parity(got[t], want[t], f"token {t}")
     shifted = moe_dev((qg, qg, qd), (0, 0, 0), mats, n_expert, n_embd, n_ff, logits, x, top_k, offset=1)
     assert np.array_equal(got, shifted)
+    # the form that ran: a workspace of the two-token form's size runs that one
+    two = moe_dev((qg, qg, qd), (0, 0, 0), mats, n_expert, n_embd, n_ff, logits, x, top_k,
+                  nb=two_token_bytes(n_tok, top_k, n_expert, n_embd, n_ff))
+    assert np.array_equal(got, two) == (tokens == 0)
 
 
 # the many-token form is taken where it is the faster one: pairs x n_embd x
@@ -112,27 +125,27 @@ def test_moe_all_tokens_on_the_same_experts(oracle):
 @pytest.mark.parametrize("quant,flags", [(Q6_K, (H.FLAG_Q6K_SIGNED_SCALES, 0, H.FLAG_Q6K_SIGNED_SCALES)),
                                          (Q6_K, (0, H.FLAG_Q6K_SIGNED_SCALES, 0)),
                                          (IQ4_XS, (H.FLAG_IQ4XS_GGML,) * 3)])
-def test_moe_many_tokens_readings(quant, flags):
-    """The flagged readings (gate's and up's may differ for Q6_K), against
-    the same tokens four at a time (moe_om.hip)."""
+def test_moe_many_tokens_readings(oracle, quant, flags):
+    """The flagged readings (gate's and up's may differ for Q6_K)."""
     print("[case] moe tokens, readings", quant, flags, flush=True)
     n_expert, n_embd, n_ff, top_k, n_tok = 16, 512, 512, 4, 40
     mats = om_tensors(n_expert, n_embd, n_ff, quant, quant, 80)
     logits = S.router_logits(81, n_tok, n_expert)
     x = S.normal_f32(82, n_tok * n_embd).reshape(n_tok, n_embd)
-    args = ((quant,) * 3, flags, mats, n_expert, n_embd, n_ff)
-    got = moe_dev(*args, logits, x, top_k)
-    for t in range(0, n_tok, 4):
-        want = moe_dev(*args, logits[t:t + 4], x[t:t + 4], top_k)
-        for i in range(4):
-            check_parity(got[t + i], want[i], f"token {t + i}", strict_tol=2 * STRICT_TOL)
+    got = moe_dev((quant,) * 3, flags, mats, n_expert, n_embd, n_ff, logits, x, top_k)
+    flagged = oracle.SCALE_I8 if quant == Q6_K else oracle.IQ4XS_GGML
+    modes = tuple(flagged if f else 0 for f in flags)
+    for t in range(n_tok):
+        ids, w = oracle.moe_route(logits[t], top_k)
+        want = oracle.moe_routed(quant, quant, quant, n_expert, n_embd, n_ff, *mats, ids, w, x[t], out_major=True,
+                                 modes=modes)
+        check_parity(got[t], want, f"token {t}")
 
 
 @pytest.mark.parametrize("n_sh,n_tok", [(256, 9), (768, 33), (512, 100)])
-def test_moe_layer_many_tokens(n_sh, n_tok):
+def test_moe_layer_many_tokens(oracle, n_sh, n_tok):
     """The whole layer (router and shared expert of many tokens in one set
-    of launches), against the same tokens four at a time; replayed from a
-    graph, eager calls between."""
+    of launches); replayed from a graph, eager calls of four tokens between."""
     import torch
     print("[case] moe layer tokens", n_sh, n_tok, flush=True)
     n_expert, n_embd, n_ff, top_k = 16, 768, 512, 6
@@ -154,12 +167,9 @@ def test_moe_layer_many_tokens(n_sh, n_tok):
     torch.cuda.synchronize()
     got = out.cpu().numpy()
     few = torch.empty((4, n_embd), device="cuda")
-    for t0 in range(0, n_tok, 4):
-        n = min(4, n_tok - t0)
-        call(t0, n, few)
-        torch.cuda.synchronize()
-        for i in range(n):
-            check_parity(got[t0 + i], few[i].cpu().numpy(), f"token {t0 + i}", strict_tol=2 * STRICT_TOL)
+    for i in range(n_tok):
+        want = oracle.moe_layer(q, t, n_expert, n_embd, n_ff, n_sh, x[i], top_k, out_major=True)
+        check_parity(got[i], want, f"token {i}")
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
         call(0, n_tok, out)
@@ -179,11 +189,10 @@ def test_moe_layer_many_tokens(n_sh, n_tok):
 
 @pytest.mark.parametrize("plain,n_expert,n_embd,n_sh,q_sh", [
     (0, 5, 768, 256, Q4_K), (0, 16, 4096, 768, Q5_K), (1, 7, 512, 4608, Q8_0), (30, 12, 2304, 256, Q6_K)])
-def test_moe_layer_one_token_front(plain, n_expert, n_embd, n_sh, q_sh):
+def test_moe_layer_one_token_front(oracle, plain, n_expert, n_embd, n_sh, q_sh):
     """One token: router, gate input and the shared expert's gate and up in
     one launch (odd and even row counts, every plain type and a row pair per
-    wave or several), against the two-token call's first token, which takes
-    them apart."""
+    wave or several), and two tokens, which take them apart."""
     import torch
     print("[case] moe layer front", plain, n_expert, n_embd, n_sh, q_sh, flush=True)
     n_ff, top_k = 256, 4
@@ -199,7 +208,7 @@ def test_moe_layer_one_token_front(plain, n_expert, n_embd, n_sh, q_sh):
     bufs = [torch.from_numpy(np.ascontiguousarray(a).reshape(-1)).cuda() for a in t]
     flags = [0, OM, OM, OM, 0, 0, 0, 0]
     tx = torch.from_numpy(x).cuda()
-    res = []
+    want = [oracle.moe_layer(q, t, n_expert, n_embd, n_ff, n_sh, x[i], top_k, out_major=True) for i in range(2)]
     for n in (1, 2):
         out = torch.full((n, n_embd), float("nan"), device="cuda")
         nb = H.moe_layer_workspace_bytes(n, top_k, n_expert, n_embd, n_ff, n_sh, q)
@@ -207,5 +216,6 @@ def test_moe_layer_one_token_front(plain, n_expert, n_embd, n_sh, q_sh):
         H.moe_layer_dev([(q[i], flags[i], bufs[i].data_ptr()) for i in range(8)], n_expert, n_embd, n_ff, n_sh, n, top_k,
                         tx.data_ptr(), out.data_ptr(), ws.data_ptr(), nb, torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
-        res.append(out.cpu().numpy()[0])
-    check_parity(res[0], res[1], "token 0", strict_tol=2 * STRICT_TOL)
+        got = out.cpu().numpy()
+        for i in range(n):
+            check_parity(got[i], want[i], f"{n} tokens, token {i}")

@@ -39,7 +39,9 @@ def test_ffn_dev_noalloc_equals_workspace_path(oracle):
     import torch
     from conftest import rel_err
     cases = [((12, 12, 12), 4096, 12288, 3),   # general path, three tokens: 2.2 MB of scratch
-             ((12, 12, 14), 2048, 4096, 1)]    # then a smaller call (mixed types)
+             ((12, 12, 14), 2048, 4096, 1),    # then a smaller call (mixed types)
+             # the many-token form: as many shares of the columns as 4 MiB hold
+             ((12, 12, 14), 4096, 12288, 17), ((12, 12, 12), 4096, 12288, 23), ((8, 8, 13), 1024, 2048, 9)]
     for quants, n_embd, n_ff, n_tok in cases:
         say("ffn noalloc", quants, n_embd, n_ff, n_tok)
         mats = [S.matrix(quants[0], 71 + n_ff, n_ff, n_embd), S.matrix(quants[1], 72 + n_ff, n_ff, n_embd),
