@@ -94,8 +94,8 @@ __device__ __forceinline__ void tok_signed4(uint32_t w, f16x2_t& a, f16x2_t& b) 
 // 64 columns (32-column sub-blocks 2g and 2g + 1), each four MFMA k steps
 // (sub-block jj, step i). load<g> issues group g's loads into Raw; take<g>
 // moves what they brought into Sb (the next super-block's loads then go into
-// Raw); frags<g, jj> forms the two B fragments of sub-block jj, and sub<g> the
-// sub-block scales of the k steps (kSub 1) or sub-blocks (kSub 2). kSub 0:
+// Raw); frags<g, jj> forms the two B fragments of sub-block jj, and sub<g> is
+// the scale of a k step (kSub 1) or sub-block (kSub 2) of the group. kSub 0:
 // the scales are in the weights. `left`: Q8_0 blocks from the super-block's
 // first to the row's last.
 // take_lds<g>: take<g> from the row's bytes in LDS (kPieces 16-byte pieces
@@ -183,7 +183,9 @@ struct TokQ4Q5 {  // Q4_K, Q5_K
     }
   }
   template <int G>
-  __device__ static __forceinline__ void sub(const Sb&, float (&)[4], int, int) {}
+  __device__ static __forceinline__ float sub(const Sb&, int, int, int) {
+    return 1.f;
+  }
 };
 
 // Q6_K: 16-element sub-blocks are the k steps. A lane half reads whole
@@ -275,19 +277,9 @@ struct TokQ6 {
     }
   }
   template <int G>
-  __device__ static __forceinline__ void sub(const Sb& s, float (&sc)[4], int q6_signed, int) {
-    const uint32_t w = G == 0 ? s.sc.x : G == 1 ? s.sc.y : G == 2 ? s.sc.z : s.sc.w;
-    if (q6_signed) {
-      sc[0] = float(int8_t(w & 0xFFu));
-      sc[1] = float(int8_t((w >> 8) & 0xFFu));
-      sc[2] = float(int8_t((w >> 16) & 0xFFu));
-      sc[3] = float(int8_t(w >> 24));
-    } else {
-      sc[0] = ubyte<0>(w);
-      sc[1] = ubyte<1>(w);
-      sc[2] = ubyte<2>(w);
-      sc[3] = ubyte<3>(w);
-    }
+  __device__ static __forceinline__ float sub(const Sb& s, int k, int q6_signed, int) {
+    const uint32_t w = (G == 0 ? s.sc.x : G == 1 ? s.sc.y : G == 2 ? s.sc.z : s.sc.w) >> (8 * k);
+    return q6_signed ? float(int8_t(w & 0xFFu)) : ubyte<0>(w);
   }
 };
 
@@ -343,9 +335,8 @@ struct TokQ8 {
     tok_signed4(q.w, f[1].h[2], f[1].h[3]);
   }
   template <int G>
-  __device__ static __forceinline__ void sub(const Sb& s, float (&sc)[4], int, int left) {
-    sc[0] = 2 * G < left ? h2f(s.d[0]) : 0.f;
-    sc[1] = 2 * G + 1 < left ? h2f(s.d[1]) : 0.f;
+  __device__ static __forceinline__ float sub(const Sb& s, int jj, int, int left) {
+    return 2 * G + jj < left ? h2f(s.d[jj]) : 0.f;
   }
 };
 
@@ -389,9 +380,8 @@ struct TokIQ4 {
     tok_signed4(iq4_lut((q.y >> 4) & 0x0F0F0F0Fu), f[1].h[2], f[1].h[3]);
   }
   template <int G>
-  __device__ static __forceinline__ void sub(const Sb& s, float (&sc)[4], int, int) {
-    sc[0] = iq4xs_scale(s.h.x, s.h.y, 2 * G);
-    sc[1] = iq4xs_scale(s.h.x, s.h.y, 2 * G + 1);
+  __device__ static __forceinline__ float sub(const Sb& s, int jj, int, int) {
+    return iq4xs_scale(s.h.x, s.h.y, 2 * G + jj);
   }
 };
 

@@ -338,8 +338,6 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
       else
         F::template frags<g, 1>(sb, f[kBoth]);
     };
-    float sc[4];
-    F::template sub<g>(sb, sc, a.q6s, left);
     auto frag_a = [&](int t, int k, int limb) {
       const int at = TOK == 8 ? (16 * half + (lane & 15)) * 16 : 16 * lane;
       return *reinterpret_cast<const f16x8_t*>(A + ((t * 4 + k) * S::kLimbs + limb) * S::kPiece + at);
@@ -369,6 +367,7 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
       // are held (the barriers keep the compiler from batching the MFMAs)
       constexpr int kSteps = F::kSub == 1 ? 1 : 2, kUnits = 4 / kSteps * NT;
       f32x16_t dd[2];
+      float sc = 0.f;
 #pragma unroll
       for (int u = 0; u <= kUnits; ++u) {
         if (u < kUnits) {
@@ -387,8 +386,9 @@ __global__ void __launch_bounds__(kTokThreads, 2) tok_mm_kernel(TokMm a) {
         }
         if (u > 0) {
           const int t = (u - 1) % NT;
+          if (t == 0) sc = F::template sub<g>(sb, (u - 1) / NT, a.q6s, left);
 #pragma unroll
-          for (int i = 0; i < kAcc; ++i) acc[t][i] = __builtin_fmaf(dd[(u - 1) & 1][i], sc[(u - 1) / NT], acc[t][i]);
+          for (int i = 0; i < kAcc; ++i) acc[t][i] = __builtin_fmaf(dd[(u - 1) & 1][i], sc, acc[t][i]);
           asm volatile("" : "+v"(acc[t]));  // here and not where the sums are used
         }
         __builtin_amdgcn_sched_barrier(0);
