@@ -24,9 +24,9 @@
 // Bound: weights are read and decoded once per group, so few tokens are
 // bound by the weight stream and many by MFMA (two f16 products per weight
 // and token). Per launch in a kernel trace: gate and up of 4096 x 12288 Q4_K
-// (two matrices) 25 us at 24 tokens, 58 us at 77, 285 us at 512 (363 TFLOP/s
-// of x, twice that of f16); down of 12288 x 4096 Q6_K 27, 44 and 244 us (its
-// 16-column sub-blocks cost 16 scalings per MFMA pair).
+// (two matrices) 25 us at 24 tokens, 58 us at 77 (MFMA 29% busy, VALU 25), 285
+// us at 512 (363 TFLOP/s of x, twice that of f16); down of 12288 x 4096 Q6_K
+// 25, 47 and 252 us (its 16-column sub-blocks cost 16 scalings per MFMA pair).
 // v_mfma_f32_32x32x16_f16: A row / B column = lane % 32, k = 8 (lane / 32) +
 // [0, 8); D column (weight row) = lane % 32, D row (token) = 8 (i / 4) + 4
 // (lane / 32) + i % 4.
@@ -195,7 +195,7 @@ constexpr bool tok_lds_format() {
 // the order they were read, and the lanes take their rows from there. Loads
 // straight to the lanes (32 rows x 32 bytes each) cost an access or two per
 // lane: Q6_K down of 96 tokens x 8 of 128 experts took 36 M accesses for 165
-// MB, and the load unit bound it. Routed FFN, 128 x 2048 x 768 Q4_K / Q6_K: 16
+// MB, and the load unit bound it; this way it takes 11. Routed FFN, 128 x 2048 x 768 Q4_K / Q6_K: 16
 // tokens 111 -> 98 us, 64 189 -> 155 to 170, 96 204 -> 169 to 186, 256 231 ->
 // 214; dense FFN
 // 2048 / 6144 Q5_K / Q8_0, 12 tokens 43 -> 34.
