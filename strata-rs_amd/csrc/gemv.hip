@@ -678,7 +678,10 @@ __device__ __forceinline__ float plain_at(const uint8_t* row, int c) {
 
 constexpr int kPlainThreads = 256, kPlainUnroll = 8;
 
-template <int Q, int NB, bool XB>
+// MANY: the vectors are NB to a blockIdx.y, the last group short; otherwise NB
+// in all, known when this is compiled (6 F32 vectors of 4096 x 4096: 24.6 us,
+// with the count at run time 26.5).
+template <int Q, int NB, bool XB, bool MANY = false>
 __global__ void __launch_bounds__(kPlainThreads) gemv_plain_kernel(const uint8_t* __restrict__ w, int rows, int cols,
                                                                   int64_t row_bytes, const float* __restrict__ x,
                                                                   float* __restrict__ y, const uint8_t* __restrict__ w2,
@@ -692,8 +695,8 @@ __global__ void __launch_bounds__(kPlainThreads) gemv_plain_kernel(const uint8_t
   const int r = tail ? int(blockIdx.x) - rows : int(blockIdx.x);
   const uint8_t* row = (tail ? w2 : w) + int64_t(r) * row_bytes;
   const bool round_x = XB && !tail;
-  // vectors NB * blockIdx.y on, `n` of them (the last repeated past that)
-  const int b0 = NB * int(blockIdx.y), n = min(NB, batch - b0);
+  // vectors b0 on, `n` of them (the last repeated past that)
+  const int b0 = MANY ? NB * int(blockIdx.y) : 0, n = MANY ? min(NB, batch - b0) : NB;
   x += int64_t(b0) * cols;
   double acc[NB];
 #pragma unroll
@@ -707,7 +710,7 @@ __global__ void __launch_bounds__(kPlainThreads) gemv_plain_kernel(const uint8_t
       wv[k] = plain_at<Q>(row, c);
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        const float v = x[int64_t(min(b, n - 1)) * cols + c];
+        const float v = x[int64_t(MANY ? min(b, n - 1) : b) * cols + c];
         xv[k][b] = round_x ? bf16_rne(v) : v;  // XB: the matvec of bf16(x)
       }
     }
@@ -802,6 +805,14 @@ static hipError_t launch_plain(int nb, const uint8_t* w, int rows, int cols, int
   // above 8 vectors: 8 to a workgroup, in one launch (a MoE layer's router,
   // 128 rows of 2048 and 96 tokens: 12 launches of 5.3 us before)
   const dim3 grid = dim3(unsigned(rows + rows2), unsigned((nb + 7) / 8)), block = dim3(kPlainThreads);
+  if (nb > 8) {  // bf16(x) alone: the matvec entry points take 8 at most
+    if constexpr (XB) {
+      hipLaunchKernelGGL((gemv_plain_kernel<Q, 8, XB, true>), grid, block, 0, s, w, rows, cols, row_bytes, x, y, w2, rows2,
+                         y2, nb);
+      return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+  }
 #define SH_PLAIN(N)                                                                                           \
   hipLaunchKernelGGL((gemv_plain_kernel<Q, N, XB>), grid, block, 0, s, w, rows, cols, row_bytes, x, y, w2, rows2, \
                      y2, nb)
